@@ -15,6 +15,7 @@
 
 #include "oxe_engine_host.h"
 #include "oxe_gemm.h"
+#include "oxe_pf_kquant.h"
 #include "oxe_prologue.h"
 #include "oxe_route.h"
 #include "oxe_shape.h"
@@ -255,18 +256,24 @@ __global__ __launch_bounds__(256) void delta_kernel(const float *cy, const float
 }
 
 // gated norm (rms_norm(o) * ssm_norm * silu(z), engine.rs:2560-2566) + Q8_0 of (token, value head),
-// one wave each
-__global__ __launch_bounds__(256) void gated_norm_kernel(const float *o, const float *proj, const float *ssm_norm, float eps,
+// one wave each; F32: the f32 values instead, over o (a K-quant output projection quantises them)
+template <bool F32>
+__global__ __launch_bounds__(256) void gated_norm_kernel(float *o, const float *proj, const float *ssm_norm, float eps,
                                                          int8_t *oq, uint16_t *od) {
     const int64_t t = blockIdx.x;
     const int vh = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const float *orow = o + t * DIN + vh * HV;
+    float *orow = o + t * DIN + vh * HV;
     const float x0 = orow[lane], x1 = orow[lane + 64];
     const float mean = wave_mean_sq_128(x0, x1, orow);
     const float sc = 1.0f / sqrtf(mean + eps);
     const float *z = proj + t * DN_ROWS + DN_Z + vh * HV;
     const float o0 = ((x0 * sc) * ssm_norm[lane]) * v_silu(z[lane]);
     const float o1 = ((x1 * sc) * ssm_norm[lane + 64]) * v_silu(z[lane + 64]);
+    if (F32) {
+        orow[lane] = o0;
+        orow[lane + 64] = o1;
+        return;
+    }
     // Q8_0 blocks of 32: lanes 0..31 hold blocks 0 (o0) and 2 (o1), lanes 32..63 blocks 1 and 3
     float d0, d1;
     const uint32_t p0 = quant32_lanes(o0, &d0), p1 = quant32_lanes(o1, &d1);
@@ -651,12 +658,17 @@ __global__ __launch_bounds__(256, 2) void attn_gqa_kernel(const uint16_t *qh, co
 // Workgroup = 16 tokens x 16 rows (row 256 is the shared gate); lane group g (16 lanes, lane = chain
 // c) holds the chains of 4 tokens x 4 rows; token and weight rows are staged through LDS 256
 // elements at a time. Every dot keeps the reference's 16 chains in order and its reduction tree.
+static_assert(DN_ALPHA == DN_BETA + NVH, "beta and alpha rows are neighbours in the projection buffer");
 constexpr int RT_TB = 16, RT_KC = 256, RT_Q = RT_KC / 16, RT_QP = RT_Q + 4, RT_NR = NEXP + 1;
 // LDS rows are stored chain-major: element 16 q + c of a stage at [row][c][q] (rows of RT_QP floats,
 // padded so that 16-byte reads of 16 consecutive chains fall on distinct banks), so a thread reads
 // four consecutive steps of its chain in one 16-byte load
+// BA: the same dots for F32 ssm_beta / ssm_alpha rows (row e < NVH of `router`, then of `shg`), into
+// the projection buffer lg where the delta-net phase reads them
+template <bool BA>
 __global__ __launch_bounds__(256) void router_kernel(const float *xn, const float *router, const float *shg, int T, float *lg,
                                                      float *sg) {
+    constexpr int NA = BA ? NVH : NEXP, NR = BA ? 2 * NVH : RT_NR;   // rows of the first matrix, of both
     __shared__ __align__(16) float s_x[RT_TB][16][RT_QP], s_w[RT_TB][16][RT_QP];
     const int tid = threadIdx.x, g = tid >> 4, c = tid & 15, tb = g & 3, eb = g >> 2;
     const int64_t t0 = (int64_t)blockIdx.x * RT_TB;
@@ -677,8 +689,8 @@ __global__ __launch_bounds__(256) void router_kernel(const float *xn, const floa
             const int64_t tt = t0 + row;
             const int ee = e0 + row;
             xr[r] = tt < T ? *(const float4 *)(xn + tt * E + k0 + 4 * c4) : make_float4(0, 0, 0, 0);
-            const float *wr = ee < NEXP ? router + (int64_t)ee * E : shg;
-            wr4[r] = ee < RT_NR ? *(const float4 *)(wr + k0 + 4 * c4) : make_float4(0, 0, 0, 0);
+            const float *wr = ee < NA ? router + (int64_t)ee * E : shg + (int64_t)(ee - NA) * E;
+            wr4[r] = ee < NR ? *(const float4 *)(wr + k0 + 4 * c4) : make_float4(0, 0, 0, 0);
         }
     };
     stage_load(0);
@@ -728,8 +740,9 @@ __global__ __launch_bounds__(256) void router_kernel(const float *xn, const floa
             if (c == 4 * i + e) mine = v[i][e];
     const int64_t tt = t0 + 4 * tb + (c >> 2);
     const int ee = e0 + 4 * eb + (c & 3);
-    if (tt < T && ee < RT_NR) {
-        if (ee < NEXP) lg[tt * NEXP + ee] = mine;
+    if (tt < T && ee < NR) {
+        if (BA) lg[tt * DN_ROWS + DN_BETA + ee] = mine;
+        else if (ee < NEXP) lg[tt * NEXP + ee] = mine;
         else sg[tt] = sigmoid_c(mine);
     }
 }
@@ -825,16 +838,21 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *dout, const i
 
 // ---- MTP entry for seeding -----------------------------------------------------------------
 // row t: [rms_norm(embd(tok)) * enorm ; rms_norm(h) * hnorm] quantised (K = 2 n_embd), as the
-// decode's entry prologue (engine.rs:2362-2390); the embedding goes to x (replay source) first
+// decode's entry prologue (engine.rs:2362-2390); the embedding goes to x (replay source) first (no
+// toks: it is already there, a K-quant embedding's rows)
 __global__ __launch_bounds__(PT) void entry_in_kernel(Q8W emb, const uint32_t *toks, const float *h, float *x,
                                                       const float *enorm, const float *hnorm, float eps, int8_t *xq,
                                                       uint16_t *xd) {
     __shared__ NormScratch ns;
     const int64_t t = blockIdx.x;
     float v[EPT];
-    embed8(emb, toks[t], v);
-    store8(x + t * E, v);
-    __syncthreads();
+    if (toks) {
+        embed8(emb, toks[t], v);
+        store8(x + t * E, v);
+        __syncthreads();
+    } else {
+        load8(x + t * E, v);
+    }
     rms_norm_mul_e(v, x + t * E, enorm, eps, ns);
     quant8(v, xq + t * 2 * E + EPT * threadIdx.x, xd + t * (2 * E / 32) + (EPT * threadIdx.x) / 32);
     const float *hr = h + t * E;
@@ -846,6 +864,16 @@ __global__ __launch_bounds__(PT) void entry_in_kernel(Q8W emb, const uint32_t *t
 }  // namespace pf
 
 // ---- host ----------------------------------------------------------------------------------------
+
+// prompts of at most this many positions of a model with K-quant / F32 matrices run as decode runs of two
+// positions (8 layers of the Ornith file's types: 2 positions 1.14 ms against 1.81 batched, 3 positions 2.28
+// against 1.57)
+constexpr int PF_KQ_RUNS = 2;
+// a K-quant matrix and the column its rows start at
+struct KqPart {
+    const RawW *r;
+    int64_t off;
+};
 
 int Engine::pf_alloc(int T) {
     if (T <= pfb.cap) return 0;
@@ -880,6 +908,18 @@ int Engine::pf_alloc(int T) {
         pfb.dout = alloc<float>(np * E);
         pfb.sh = alloc<float>((size_t)T * E);
         pfb.tok = alloc<uint32_t>((size_t)T);
+        if (kq) {
+            auto act = [&](size_t rows, size_t k) {
+                KqAct a;
+                a.c16 = alloc<uint16_t>(rows * k);
+                a.c8 = alloc<int8_t>(rows * k);
+                a.d = alloc<float>(rows * (k / 256));
+                a.bs = alloc<uint16_t>(rows * (k / 16));
+                return a;
+            };
+            pfb.ka = act(T, MIX_W);
+            pfb.kh = act(np, FF);
+        }
         pfb.cap = T;
     } catch (...) {
         set_err("out of device memory for the prefill buffers");
@@ -942,12 +982,62 @@ int Engine::pf_chunk(const uint32_t *toks, int T, float *h_out) {
         probe(K_PF_EXPERT); probe(K_PF_GEMM);
         return r;
     };
+    // K-quant matrices of k columns over the activation a: consecutive parts of one type share a launch
+    auto kgemm = [&](const KqPart *ps, int n, int64_t k, const KqAct &a, float *y, int64_t ldy, const float *res, int64_t nt,
+                     const int32_t *xrow, bool grp) {
+        for (int i = 0, e; i < n; i = e) {
+            KqGemmArgs g{};
+            for (e = i; e < n && e - i < KQG_SEGS && ps[e].r->type == ps[i].r->type; e++)
+                g.seg[g.nseg++] = KqGemmSeg{ps[e].r->w, ps[e].r->rows, ps[e].off, ps[e].r->rows * raw_row_bytes(*ps[e].r)};
+            g.nb = (int)(k / 256);
+            g.x = a; g.y = y; g.ldy = ldy; g.res = res; g.ldr = res ? E : 0; g.nt = nt; g.xrow = xrow;
+            if (grp) {
+                g.tiles = pfb.tiles;
+                g.tile_count = pfb.mo + MO_NT;
+            }
+            probe(K_PF_GEMM);
+            if (grp) probe(K_PF_EXPERT);
+            const int r = kq_gemm_launch(ps[i].r->type, g, grp ? pfb.max_tiles : 0, st);
+            if (grp) probe(K_PF_EXPERT);
+            probe(K_PF_GEMM);
+            if (r) return r;
+        }
+        return 0;
+    };
+    // the forms of a's codes that the parts' types read
+    auto forms = [](const KqAct &a, const KqPart *ps, int n) {
+        bool f16 = false, i8 = false;
+        for (int i = 0; i < n; i++)
+            if (ps[i].r->type >= 11) (kqg_f16(ps[i].r->type) ? f16 : i8) = true;
+        KqAct r = a;
+        if (!f16) r.c16 = nullptr;
+        if (!i8) r.c8 = nullptr;
+        return r;
+    };
     for (int il = 0; il < d.n_layer; il++) {
         const LayerW &w = L[il];
+        const bool kproj = w.kq_proj(), kout = w.out_r.type != 8, ba32 = !w.att && w.beta_r.type == 0;
+        const bool kemb = il == 0 && m.tok_embd_r.type != 8;
+        if (kemb && (rc = kq_pf_embed(m.tok_embd_r, pfb.tok, T, pfb.x, st))) return rc;
         // input norm + Q8_0 (layer 0: the token embeddings, also the residual)
-        hipLaunchKernelGGL(norm_quant_kernel, dim3(T), dim3(PT), 0, st, m.tok_embd, il == 0 ? pfb.tok : nullptr, pfb.x,
-                           w.attn_norm, eps, pfb.xq, pfb.xd, (int64_t)E, nullptr);
-        if ((rc = gemm(w.proj, pfb.xq, pfb.xd, E, pfb.proj, DN_ROWS, nullptr, T))) return rc;
+        hipLaunchKernelGGL(norm_quant_kernel, dim3(T), dim3(PT), 0, st, m.tok_embd, il == 0 && !kemb ? pfb.tok : nullptr, pfb.x,
+                           w.attn_norm, eps, pfb.xq, pfb.xd, (int64_t)E, kproj || ba32 ? pfb.xn : nullptr);
+        if (kproj) {
+            const KqPart dn[4] = {{&w.qkv_r, 0}, {&w.z_r, DN_Z}, {&w.beta_r, DN_BETA}, {&w.alpha_r, DN_ALPHA}};
+            const KqPart at[3] = {{&w.q_r, 0}, {&w.k_r, AT_K}, {&w.v_r, AT_V}};
+            const KqPart *ps = w.att ? at : dn;
+            const int n = w.att ? 3 : ba32 ? 2 : 4;
+            const KqAct a = forms(pfb.ka, ps, n);
+            if ((rc = kq_pf_quant(pfb.xn, E, T, E, a, st))) return rc;
+            if ((rc = kgemm(ps, n, E, a, pfb.proj, DN_ROWS, nullptr, T, nullptr, false))) return rc;
+        } else {
+            Q8W p = w.proj;
+            if (ba32) p.rows = DN_BETA;
+            if ((rc = gemm(p, pfb.xq, pfb.xd, E, pfb.proj, DN_ROWS, nullptr, T))) return rc;
+        }
+        if (ba32)
+            hipLaunchKernelGGL(router_kernel<true>, dim3((T + RT_TB - 1) / RT_TB, 2 * NVH / RT_TB), dim3(256), 0, st, pfb.xn,
+                               (const float *)w.beta_r.w, (const float *)w.alpha_r.w, T, pfb.proj, nullptr);
         if (!w.att) {
             float *cs = m.conv_state + (int64_t)cur * conv_slot + (int64_t)w.index * NCH * (KC - 1);
             float *ss = m.ssm_state + (int64_t)cur * ssm_slot + (int64_t)w.index * NVH * HV * HV;
@@ -958,8 +1048,12 @@ int Engine::pf_chunk(const uint32_t *toks, int T, float *h_out) {
             probe(K_PF_DELTA);
             hipLaunchKernelGGL(delta_kernel, dim3(NVH * 8), dim3(256), 0, st, pfb.cy, pfb.gg, pfb.gb, ss, pfb.o, T);
             probe(K_PF_DELTA);
-            hipLaunchKernelGGL(gated_norm_kernel, dim3(T, NVH / 4), dim3(256), 0, st, pfb.o, pfb.proj, w.ssm_norm, eps,
-                               pfb.oq, pfb.od);
+            if (kout)
+                hipLaunchKernelGGL(gated_norm_kernel<true>, dim3(T, NVH / 4), dim3(256), 0, st, pfb.o, pfb.proj, w.ssm_norm, eps,
+                                   nullptr, nullptr);
+            else
+                hipLaunchKernelGGL(gated_norm_kernel<false>, dim3(T, NVH / 4), dim3(256), 0, st, pfb.o, pfb.proj, w.ssm_norm,
+                                   eps, pfb.oq, pfb.od);
         } else {
             uint16_t *kcl = m.kcache + (int64_t)w.index * NKV * n_ctx * HD;
             uint16_t *vtl = m.vcache + (int64_t)w.index * NKV * HD * n_ctx;
@@ -973,30 +1067,67 @@ int Engine::pf_chunk(const uint32_t *toks, int T, float *h_out) {
                 hipLaunchKernelGGL(attn_kernel, dim3(T, NH), dim3(256), (size_t)kv_cap * 6, st, pfb.qh, kcl, vtl, pfb.proj,
                                    p0, n_ctx, kv_cap, pfb.o);
             probe(K_PF_ATTN);
-            if ((rc = quantize_q8_0(pfb.o, (int64_t)T * MIX_W, pfb.oq, pfb.od, st))) return rc;
+            if (!kout && (rc = quantize_q8_0(pfb.o, (int64_t)T * MIX_W, pfb.oq, pfb.od, st))) return rc;
         }
         // mixer output projection + residual
-        if ((rc = gemm(w.out, pfb.oq, pfb.od, MIX_W, pfb.x1, E, pfb.x, T))) return rc;
+        if (kout) {
+            const KqPart ps[1] = {{&w.out_r, 0}};
+            const KqAct a = forms(pfb.ka, ps, 1);
+            if ((rc = kq_pf_quant(pfb.o, MIX_W, T, MIX_W, a, st))) return rc;
+            if ((rc = kgemm(ps, 1, MIX_W, a, pfb.x1, E, pfb.x, T, nullptr, false))) return rc;
+        } else if ((rc = gemm(w.out, pfb.oq, pfb.od, MIX_W, pfb.x1, E, pfb.x, T))) {
+            return rc;
+        }
         // post-attention norm: Q8_0 for the experts, f32 for the router
         hipLaunchKernelGGL(norm_quant_kernel, dim3(T), dim3(PT), 0, st, m.tok_embd, nullptr, pfb.x1, w.post_norm, eps,
                            pfb.xq, pfb.xd, (int64_t)E, pfb.xn);
-        hipLaunchKernelGGL(router_kernel, dim3((T + RT_TB - 1) / RT_TB, (RT_NR + RT_TB - 1) / RT_TB), dim3(256), 0, st,
+        hipLaunchKernelGGL(router_kernel<false>, dim3((T + RT_TB - 1) / RT_TB, (RT_NR + RT_TB - 1) / RT_TB), dim3(256), 0, st,
                            pfb.xn, w.router, w.shexp_gate, T, pfb.lg, pfb.sg);
         hipLaunchKernelGGL(route_kernel, dim3((T + 3) / 4), dim3(256), 0, st, pfb.lg, T, pfb.ids, pfb.wts,
                            b.counters + CNT_ERR_TIE);
+        // gate / up as [gate | up] columns from K-quant matrices, interleaved 8 by 8 from a Q8_0 one
+        const KqPart egu[2] = {{&w.exp_gate_r, 0}, {&w.exp_up_r, FF}}, sgu[2] = {{&w.sh_gate_r, 0}, {&w.sh_up_r, FFSH}};
+        const KqPart edn[1] = {{&w.exp_down_r, 0}}, sdn[1] = {{&w.sh_down_r, 0}};
+        const bool kegu = w.exp_gate_r.type != 8, ksgu = w.sh_gate_r.type != 8;
+        const bool kedn = w.exp_down_r.type != 8, ksdn = w.sh_down_r.type != 8;
+        KqAct xa{};
+        if (kegu || ksgu) {
+            const KqPart all[4] = {egu[0], egu[1], sgu[0], sgu[1]};
+            xa = forms(pfb.ka, all, 4);
+            if ((rc = kq_pf_quant(pfb.xn, E, T, E, xa, st))) return rc;
+        }
+        // swiglu of `rows` gate / up rows, quantised as the down matrix reads h
+        auto swiglu = [&](bool split, const KqPart *dn, int64_t rows, KqAct &h) {
+            if (dn->r->type != 8) {
+                h = forms(pfb.kh, dn, 1);
+                return kq_pf_swiglu_q8_K(pfb.gu, split, rows, h, st);
+            }
+            if (split) return kq_pf_swiglu_q8_0(pfb.gu, true, rows, pfb.hq, pfb.hd, st);
+            hipLaunchKernelGGL(swiglu_quant_kernel, dim3((unsigned)rows), dim3(256), 0, st, pfb.gu, pfb.hq, pfb.hd);
+            return 0;
+        };
+        KqAct h{};
         // shared expert over all tokens
-        if ((rc = gemm(w.shexp_gu, pfb.xq, pfb.xd, E, pfb.gu, 2 * FFSH, nullptr, T))) return rc;
-        hipLaunchKernelGGL(swiglu_quant_kernel, dim3(T), dim3(256), 0, st, pfb.gu, pfb.hq, pfb.hd);
-        if ((rc = gemm(w.shexp_down, pfb.hq, pfb.hd, FFSH, pfb.sh, E, nullptr, T))) return rc;
+        if (ksgu) rc = kgemm(sgu, 2, E, xa, pfb.gu, 2 * FFSH, nullptr, T, nullptr, false);
+        else rc = gemm(w.shexp_gu, pfb.xq, pfb.xd, E, pfb.gu, 2 * FFSH, nullptr, T);
+        if (rc) return rc;
+        if ((rc = swiglu(ksgu, sdn, T, h))) return rc;
+        if (ksdn) rc = kgemm(sdn, 1, FFSH, h, pfb.sh, E, nullptr, T, nullptr, false);
+        else rc = gemm(w.shexp_down, pfb.hq, pfb.hd, FFSH, pfb.sh, E, nullptr, T);
+        if (rc) return rc;
         // routed experts: pairs grouped by expert, 64-pair tiles built on the device
         if (hipMemsetAsync(pfb.mo, 0, NEXP * 4, st) != hipSuccess) return -2;
         hipLaunchKernelGGL(moe_count_kernel, dim3((np + 255) / 256), dim3(256), 0, st, pfb.ids, np, pfb.mo);
         hipLaunchKernelGGL(moe_tiles_kernel, dim3(1), dim3(NEXP), 0, st, pfb.mo, pfb.tiles);
         hipLaunchKernelGGL(moe_scatter_kernel, dim3((np + 255) / 256), dim3(256), 0, st, pfb.ids, np, pfb.mo, pfb.ptok,
                            pfb.pair_of);
-        if ((rc = grouped(w.exp_gu, 2 * FF, E, pfb.xq, pfb.xd, pfb.ptok, pfb.gu))) return rc;
-        hipLaunchKernelGGL(swiglu_quant_kernel, dim3(np), dim3(256), 0, st, pfb.gu, pfb.hq, pfb.hd);
-        if ((rc = grouped(w.exp_down, E, FF, pfb.hq, pfb.hd, nullptr, pfb.dout))) return rc;
+        if (kegu) rc = kgemm(egu, 2, E, xa, pfb.gu, 2 * FF, nullptr, T, pfb.ptok, true);
+        else rc = grouped(w.exp_gu, 2 * FF, E, pfb.xq, pfb.xd, pfb.ptok, pfb.gu);
+        if (rc) return rc;
+        if ((rc = swiglu(kegu, edn, np, h))) return rc;
+        if (kedn) rc = kgemm(edn, 1, FF, h, pfb.dout, E, nullptr, np, nullptr, true);
+        else rc = grouped(w.exp_down, E, FF, pfb.hq, pfb.hd, nullptr, pfb.dout);
+        if (rc) return rc;
         hipLaunchKernelGGL(combine_kernel, dim3((unsigned)(((int64_t)T * E + 255) / 256)), dim3(256), 0, st, pfb.dout,
                            pfb.pair_of, pfb.wts, pfb.sh, pfb.sg, pfb.x1, pfb.x, T);
         if (hipGetLastError() != hipSuccess) return -2;
@@ -1005,9 +1136,13 @@ int Engine::pf_chunk(const uint32_t *toks, int T, float *h_out) {
     hipLaunchKernelGGL(norm_quant_kernel, dim3(T), dim3(PT), 0, st, m.tok_embd, nullptr, pfb.x, m.out_norm, eps, pfb.xq,
                        pfb.xd, (int64_t)E, pfb.xn);
     // the LM head of one token is a weight stream: the lane GEMV (HBM-bound), not the GEMM
-    rc = oxe_hip_gemv_q8_0(E, m.output.rows, 1, m.output.q, m.output.d, pfb.xq + (int64_t)(T - 1) * E,
-                           pfb.xd + (int64_t)(T - 1) * (E / 32), b.logits, nullptr, st);
-    if (rc != 1) return rc == 0 ? -1 : rc;   // 1: done (oxe_vl_gemv's convention)
+    if (m.output_r.type != 8) {
+        if ((rc = kq_head_one(m.output_r, pfb.xn + (int64_t)(T - 1) * E, b.xk, b.logits, st))) return rc;
+    } else {
+        rc = oxe_hip_gemv_q8_0(E, m.output.rows, 1, m.output.q, m.output.d, pfb.xq + (int64_t)(T - 1) * E,
+                               pfb.xd + (int64_t)(T - 1) * (E / 32), b.logits, nullptr, st);
+        if (rc != 1) return rc == 0 ? -1 : rc;   // 1: done (oxe_vl_gemv's convention)
+    }
     if (hipMemcpyAsync(b.hid, pfb.xn + (int64_t)(T - 1) * E, (size_t)E * 4, hipMemcpyDeviceToDevice, st) != hipSuccess)
         return -2;
     if (h_out && hipMemcpyAsync(h_out, pfb.xn, (size_t)T * E * 4, hipMemcpyDeviceToHost, st) != hipSuccess) return -2;
@@ -1018,9 +1153,9 @@ int Engine::pf_chunk(const uint32_t *toks, int T, float *h_out) {
 
 int Engine::prefill(const uint32_t *toks, int n, uint32_t *next, float *h_all) {
     if (n < 1 || pos + n > m.n_ctx || !toks_ok(toks, n)) return -1;
-    if (kq) {
-        // the batched pass's GEMMs take Q8_0 matrices: a model with K-quant / F32 matrices runs the
-        // decode runs two positions at a time (every position's state and h_nextn are the same)
+    if (kq && n <= PF_KQ_RUNS) {
+        // a few positions of a model with K-quant / F32 matrices: decode runs of two positions (every
+        // position's state and h_nextn are the batched pass's)
         uint32_t g[OXE_NL] = {};
         for (int c0 = 0; c0 < n; c0 += OXE_NL) {
             const int c = std::min(OXE_NL, n - c0);
@@ -1030,7 +1165,15 @@ int Engine::prefill(const uint32_t *toks, int n, uint32_t *next, float *h_all) {
             for (int i = 0; i < c && h_all; i++)
                 if ((rc = hidden_host(i, h_all + (size_t)(c0 + i) * E))) return rc;
         }
-        if (next) *next = g[(n - 1) % OXE_NL];
+        const int last = (n - 1) % OXE_NL;   // the last token's lane: its row is lane 0's after a prefill
+        if (last) {
+            if (hipMemcpyAsync(b.logits, b.logits + (size_t)last * d.n_vocab, (size_t)d.n_vocab * 4, hipMemcpyDeviceToDevice,
+                               st) != hipSuccess ||
+                hipMemcpyAsync(b.hid, b.hid + (size_t)last * E, (size_t)E * 4, hipMemcpyDeviceToDevice, st) != hipSuccess ||
+                hipStreamSynchronize(st) != hipSuccess)
+                return -2;
+        }
+        if (next) *next = g[last];
         return 0;
     }
     int rc = pf_alloc(std::min(n, PF_CHUNK));
@@ -1061,16 +1204,7 @@ int Engine::seed_batched(const uint32_t *toks, int n, int pos0, const float *hs)
     using namespace pf;
     if (n < 1 || pos0 < 0 || pos0 + n > m.n_ctx || !toks_ok(toks, n) || !hs) return -1;
     const LayerW &w = L[d.n_layer];
-    if (m.tok_embd_r.type != 8 || w.kq_proj()) {
-        // the batched kernels below read the Q8_0 token embedding and the MTP layer's Q8_0
-        // projection; a model with either in other blocks seeds through the seeding runs, OXE_NL
-        // pairs at a time (every pair's K / V rows depend on that pair only)
-        for (int c0 = 0; c0 < n; c0 += OXE_NL) {
-            const int c = std::min(OXE_NL, n - c0);
-            if (int rc = mtp_seed(toks + c0, c, pos0 + c0, hs + (size_t)c0 * E)) return rc;
-        }
-        return 0;
-    }
+    const bool kemb = m.tok_embd_r.type != 8, kproj = w.kq_proj();
     int rc = pf_alloc(std::min(n, PF_CHUNK));
     if (rc) return rc;
     uint16_t *kcl = m.kcache + (int64_t)w.index * NKV * m.n_ctx * HD;
@@ -1080,19 +1214,30 @@ int Engine::seed_batched(const uint32_t *toks, int n, int pos0, const float *hs)
         if (hipMemcpyAsync(pfb.tok, toks + c0, (size_t)T * 4, hipMemcpyHostToDevice, st) != hipSuccess) return -2;
         if (hipMemcpyAsync(pfb.hin, hs + (size_t)c0 * E, (size_t)T * E * 4, hipMemcpyHostToDevice, st) != hipSuccess)
             return -2;
-        hipLaunchKernelGGL(entry_in_kernel, dim3(T), dim3(PT), 0, st, m.tok_embd, pfb.tok, pfb.hin, pfb.x, w.enorm, w.hnorm,
-                           m.eps, pfb.xq, pfb.xd);
+        if (kemb && (rc = kq_pf_embed(m.tok_embd_r, pfb.tok, T, pfb.x, st))) return rc;
+        hipLaunchKernelGGL(entry_in_kernel, dim3(T), dim3(PT), 0, st, m.tok_embd, kemb ? nullptr : pfb.tok, pfb.hin, pfb.x,
+                           w.enorm, w.hnorm, m.eps, pfb.xq, pfb.xd);
         GemmArgs g{};
         g.wq = w.eh_proj.q; g.wd = w.eh_proj.d; g.xq = pfb.xq; g.xd = pfb.xd; g.y = pfb.x1;
         g.nr = E; g.nt = T; g.k = 2 * E; g.ldy = E;
         if ((rc = gemm_launch(g, 0, st))) return rc;
         hipLaunchKernelGGL(norm_quant_kernel, dim3(T), dim3(PT), 0, st, m.tok_embd, nullptr, pfb.x1, w.attn_norm, m.eps,
-                           pfb.xq, pfb.xd, (int64_t)E, nullptr);
-        GemmArgs k{};
-        k.wq = w.proj.q + (int64_t)AT_K * E; k.wd = w.proj.d + (int64_t)AT_K * (E / 32);
-        k.xq = pfb.xq; k.xd = pfb.xd; k.y = pfb.proj + AT_K;
-        k.nr = AT_ROWS - AT_K; k.nt = T; k.k = E; k.ldy = DN_ROWS;
-        if ((rc = gemm_launch(k, 0, st))) return rc;
+                           pfb.xq, pfb.xd, (int64_t)E, kproj ? pfb.xn : nullptr);
+        if (kproj) {
+            if ((rc = kq_pf_quant(pfb.xn, E, T, E, pfb.ka, st))) return rc;
+            for (const KqPart &p : {KqPart{&w.k_r, AT_K}, KqPart{&w.v_r, AT_V}}) {
+                KqGemmArgs k{};
+                k.seg[0] = KqGemmSeg{p.r->w, p.r->rows, p.off, 0};
+                k.nseg = 1; k.nb = E / 256; k.x = pfb.ka; k.y = pfb.proj; k.ldy = DN_ROWS; k.nt = T;
+                if ((rc = kq_gemm_launch(p.r->type, k, 0, st))) return rc;
+            }
+        } else {
+            GemmArgs k{};
+            k.wq = w.proj.q + (int64_t)AT_K * E; k.wd = w.proj.d + (int64_t)AT_K * (E / 32);
+            k.xq = pfb.xq; k.xd = pfb.xd; k.y = pfb.proj + AT_K;
+            k.nr = AT_ROWS - AT_K; k.nt = T; k.k = E; k.ldy = DN_ROWS;
+            if ((rc = gemm_launch(k, 0, st))) return rc;
+        }
         hipLaunchKernelGGL(attn_prep_kernel, dim3(T, 5), dim3(256), 0, st, pfb.proj, w.q_norm, w.k_norm, m.rope,
                            pos0 + c0, m.eps, pfb.qh, kcl, vtl, m.n_ctx, 1);
     }

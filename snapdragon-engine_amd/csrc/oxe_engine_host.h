@@ -16,6 +16,7 @@
 #include "oxe_kernels.h"
 #include "oxe_fused.h"
 #include "oxe_model_kernels.h"
+#include "oxe_pf_kquant.h"
 #include "oxe_shape.h"
 
 #define OXE_HOST_DEV_INLINE __host__ __device__ inline
@@ -63,6 +64,7 @@ struct PfBufs {
     int32_t *ids, *mo, *ptok, *pair_of;
     int4 *tiles;
     uint32_t *tok;
+    KqAct ka, kh;   // q8_K activations and expert h (a model with K-quant matrices)
 };
 constexpr int PF_CHUNK = 2048;   // tokens per batched pass
 
@@ -83,7 +85,7 @@ struct Engine {
     ModelRt m{};
     std::vector<LayerW> L;  // n_layer (+1 MTP block)
     ModelTypes types;       // the matrices' types
-    bool kq = false;        // some matrix is not Q8_0: per-phase runs, token-by-token prefill
+    bool kq = false;        // some matrix is not Q8_0: per-phase runs
     ActBufs b{};
     RunCtl *ctl = nullptr;  // device
     // the device-driven step's draft control block (fused runs), filled by the previous step's
