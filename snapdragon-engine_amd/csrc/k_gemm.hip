@@ -241,6 +241,230 @@ __global__ __launch_bounds__(gm::NT, 3) void gemm_q8_kernel(GemmArgs a, int vec4
     }
 }
 
+// ---- few tokens -------------------------------------------------------------------------------------
+// The same products where the tiles above leave the chip idle (a short prompt: 2048 rows x 45 tokens are
+// 16 workgroups, each walking K alone one stage ahead): one wave per TS x TS output tile, TS 16 or 32. A
+// wave loads its rows' and tokens' blocks, four at a time, as whole 128-byte lines (8 rows a load) into
+// registers, RD stages ahead, and turns each stage into fragments through LDS of its own: no barrier, and a
+// wait for a stage leaves the later ones in flight. Fragments read straight from global memory, 16 or 32
+// rows of 32 bytes a load, took about 4 cycles of the CU's load path per row; direct global-to-LDS loads
+// about 190 cycles each for a lone wave. Scale products of four (TS 16) or two (TS 32) blocks come from one
+// rank-1 matrix product: lane group g holds the scale of block b + g. The chain of an output is the one
+// above. Bound by the latency of a stage's steps in a lone wave (LDS, matrix product, chain).
+// K 4096 x 2048 rows, 45 tokens: 38.3 us by the large tile, 10.5 us.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// LDS accesses of this wave before it come before those after it (one wave: the LDS runs them in order)
+__device__ __forceinline__ void lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int TS>
+struct SmallStage {
+    static constexpr int RD = TS == 16 ? 6 : 3;                 // stages in flight
+    static constexpr int BYTES = 2 * TS * 128 + 2 * TS * 8;     // codes of both operands, their scales
+};
+
+template <int TS>
+__global__ __launch_bounds__(64) void gemm_q8_small_kernel(GemmArgs a, int vec4) {
+    using R = SmallStage<TS>;
+    constexpr int NG = 64 / TS;            // lanes per row: 4 of 8 bytes, or 2 of 16 bytes, per block
+    constexpr int NV = TS * TS / 64;       // outputs per lane
+    constexpr int NS = 4 / NG;             // scale products per stage of four blocks
+    typedef typename std::conditional<TS == 16, u32x2, u32x4>::type frag_t;
+    __shared__ __align__(16) int8_t sm[R::BYTES];   // one stage
+    const int lane = threadIdx.x, fr = lane & (TS - 1), g = lane / TS;
+    const int64_t k = a.k, nr = a.nr, nb = k / 32;
+    const int64_t p0 = (int64_t)blockIdx.y * TS;
+    int64_t pn = a.nt - p0;
+    if (pn > TS) pn = TS;
+    const int64_t r0 = (int64_t)blockIdx.x * TS;
+    // rows past the matrix, tokens past the tile: a valid one, never stored
+    auto wrow = [&](int i) { return r0 + i < nr ? r0 + i : nr - 1; };
+    auto xrow = [&](int i) -> int64_t {
+        const int64_t p = p0 + (i < pn ? i : 0);
+        return a.xrow ? (int64_t)a.xrow[p] : p;
+    };
+    // code loads: lane L of load q fills row 8 q + (L >> 3), slot L & 7 with chunk (L & 7) ^ f(row);
+    // scale loads: f16 pair L & 1 of row L >> 1 (TS 16: the weights' rows, then the tokens')
+    const int lr8 = lane >> 3;
+    uint32_t wofs[TS / 8], xofs[TS / 8], sofs[2 * TS / 32];
+#pragma unroll
+    for (int q = 0; q < TS / 8; q++) {
+        const uint32_t c = 16 * ((lane & 7) ^ lr8 ^ (q & 1));
+        wofs[q] = (uint32_t)(wrow(8 * q + lr8) * k) + c;
+        xofs[q] = (uint32_t)(xrow(8 * q + lr8) * k) + c;
+    }
+    const int srow = lane >> 1;
+    const bool sx = TS == 16 && lane >= 32;
+    if constexpr (TS == 16) {
+        sofs[0] = (uint32_t)((sx ? xrow(srow - 16) : wrow(srow)) * nb * 2 + 4 * (lane & 1));
+    } else {
+        sofs[0] = (uint32_t)(wrow(srow) * nb * 2 + 4 * (lane & 1));
+        sofs[1] = (uint32_t)(xrow(srow) * nb * 2 + 4 * (lane & 1));
+    }
+    const int8_t *wq = a.wq, *wsb = (const int8_t *)a.wd, *xsb = (const int8_t *)a.xd;
+    const int8_t *sb0 = TS == 16 && sx ? xsb : wsb;
+    struct Stage {
+        u32x4 w[TS / 8], x[TS / 8];
+        uint32_t s[2 * TS / 32];
+    } st[R::RD];
+    auto fetch = [&](Stage &G, int64_t i) {
+        const int8_t *wb = wq + 128 * i, *xb = a.xq + 128 * i;
+#pragma unroll
+        for (int q = 0; q < TS / 8; q++) G.w[q] = *(const u32x4 *)(wb + wofs[q]);
+#pragma unroll
+        for (int q = 0; q < TS / 8; q++) G.x[q] = *(const u32x4 *)(xb + xofs[q]);
+        G.s[0] = *(const uint32_t *)(sb0 + 8 * i + sofs[0]);
+        if constexpr (TS == 32) G.s[1] = *(const uint32_t *)(xsb + 8 * i + sofs[1]);
+    };
+    auto put = [&](const Stage &G) {
+#pragma unroll
+        for (int q = 0; q < TS / 8; q++) *(u32x4 *)(sm + 1024 * q + 16 * lane) = G.w[q];
+#pragma unroll
+        for (int q = 0; q < TS / 8; q++) *(u32x4 *)(sm + TS * 128 + 1024 * q + 16 * lane) = G.x[q];
+        *(uint32_t *)(sm + 2 * TS * 128 + 4 * lane) = G.s[0];
+        if constexpr (TS == 32) *(uint32_t *)(sm + 2 * TS * 128 + 256 + 4 * lane) = G.s[1];
+    };
+    float acc[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) acc[v] = 0.0f;
+    const int sw = (fr & 7) ^ ((fr >> 3) & 1);
+    // a stage's fragments in registers; NG blocks' dots and scale products (one rank-1 product)
+    struct Frag {
+        frag_t w[4], x[4];
+        uint16_t dw[NS], dx[NS];
+    };
+    struct Dots {
+        int32_t s[NG][NV];
+        float d[NG * NV];
+    };
+    auto read = [&](Frag &F) {
+        const int8_t *S = sm;
+        const uint16_t *sd = (const uint16_t *)(S + 2 * TS * 128);
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            F.dw[s] = sd[4 * fr + NG * s + g];
+            F.dx[s] = sd[4 * (TS + fr) + NG * s + g];
+        }
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            // lane group g of a row: bytes 8 g .. (TS 16) or 16 g .. (TS 32) of the block
+            const int at = fr * 128 + (TS == 16 ? 16 * ((2 * b + (g >> 1)) ^ sw) + 8 * (g & 1) : 16 * ((2 * b + g) ^ sw));
+            F.w[b] = *(const frag_t *)(S + at);
+            F.x[b] = *(const frag_t *)(S + TS * 128 + at);
+        }
+    };
+    auto dots = [&](const Frag &F, int s, Dots &D) {
+        const float dw = h2f(F.dw[s]), dx = h2f(F.dx[s]);
+        if constexpr (TS == 16) {
+            const f32x16 zero = {};
+            const f32x16 t = __builtin_amdgcn_mfma_f32_16x16x1f32(dw, dx, zero, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < NG * NV; v++) D.d[v] = t[v];
+        } else {
+            const f32x32 zero = {};
+            const f32x32 t = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, dx, zero, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < NG * NV; v++) D.d[v] = t[v];
+        }
+#pragma unroll
+        for (int b = 0; b < NG; b++) {
+            if constexpr (TS == 16) {
+                const i32x4 zero = {};
+                const i32x4 t = __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, F.w[NG * s + b]),
+                                                                     __builtin_bit_cast(long, F.x[NG * s + b]), zero, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < NV; v++) D.s[b][v] = t[v];
+            } else {
+                const i32x16 zero = {};
+                const i32x16 t = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, F.w[NG * s + b]),
+                                                                      __builtin_bit_cast(i32x4, F.x[NG * s + b]), zero, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < NV; v++) D.s[b][v] = t[v];
+            }
+        }
+    };
+    auto chain = [&](const Dots &D) {
+#pragma unroll
+        for (int b = 0; b < NG; b++)
+#pragma unroll
+            for (int v = 0; v < NV; v++) acc[v] = __builtin_fmaf((float)D.s[b][v], D.d[NV * b + v], acc[v]);
+    };
+    const int ng = (int)(k / 128);
+#pragma unroll
+    for (int j = 0; j < R::RD; j++) {
+        fetch(st[j], j < ng ? j : ng - 1);
+        __builtin_amdgcn_sched_barrier(0);   // stage by stage, so that a wait covers its own stage only
+    }
+    // the next stage's fragments are on their way from LDS while the chain runs over the current dots
+    Frag F;
+    Dots D[NS];
+    auto take = [&](Stage &G, int i) {
+        lds_fence();   // the previous stage's reads come before these writes
+        put(G);
+        fetch(G, i + R::RD < ng ? i + R::RD : ng - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        lds_fence();
+        read(F);
+        __builtin_amdgcn_sched_barrier(0);   // every read on its way before the chain
+    };
+    take(st[0], 0);
+#pragma unroll
+    for (int s = 0; s < NS; s++) dots(F, s, D[s]);
+    for (int i = 0; i < ng; i += R::RD) {
+#pragma unroll
+        for (int j = 0; j < R::RD; j++) {
+            const int at = i + j;   // chain of stage at, dots of stage at + 1
+            if (at >= ng) break;
+            take(st[(j + 1) % R::RD], at + 1);
+#pragma unroll
+            for (int s = 0; s < NS; s++) {
+                chain(D[s]);
+                dots(F, s, D[s]);
+            }
+        }
+    }
+    if (fr >= pn) return;
+    // outputs of a lane: token fr, rows 8 q + 4 g + e (TS 32, v = 4 q + e) or 4 g + e (TS 16)
+    const int64_t p = p0 + fr;
+    float *yp = a.y + p * a.ldy;
+    const float *rp = a.res ? a.res + p * a.ldr : nullptr;
+#pragma unroll
+    for (int q = 0; q < NV / 4; q++) {
+        const int64_t gr0 = r0 + 8 * q + 4 * g;
+        float o[4] = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+        if (vec4 && gr0 + 3 < nr) {
+            if (rp) {
+                const float4 r4 = *(const float4 *)(rp + gr0);
+                o[0] += r4.x; o[1] += r4.y; o[2] += r4.z; o[3] += r4.w;
+            }
+            *(float4 *)(yp + gr0) = make_float4(o[0], o[1], o[2], o[3]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (gr0 + e < nr) yp[gr0 + e] = rp ? o[e] + rp[gr0 + e] : o[e];
+        }
+    }
+}
+
+// The tile of a plain GEMM: 16, 32 (one wave each) or 0 (the 128 x 64 workgroup tile). Time of one round of
+// tiles at K 4096: 10 us (16), 21 us (32), 38 us (128 x 64, 768 of them resident); a round is about 600 wave tiles (more share
+// a CU's load path). Measured, few tokens against the large tile (us): [2048 x 4096] 45 tokens 10.5 / 38, 200: 20 / 39, 701:
+// 45 / 40 (stays large); [1024 x 2048] 64: 6.4 / 21.6, 701: 14.7 / 22.6; [12352 x 2048] 3: 9.8 / 18, 64: 17 / 23,
+// 100: 28 / 24 (stays large).
+static int small_tile(int64_t nr, int64_t nt) {
+    auto rounds = [](int64_t tiles, int64_t per) { return tiles > per ? (double)tiles / (double)per : 1.0; };
+    auto tiles = [&](int64_t r, int64_t t) { return ((nr + r - 1) / r) * ((nt + t - 1) / t); };
+    const double c16 = 10.0 * rounds(tiles(16, 16), 600), c32 = 21.0 * rounds(tiles(32, 32), 600);
+    const double big = 38.0 * rounds(tiles(gm::BM, gm::BN), 768);
+    return c16 <= c32 && c16 < big ? 16 : c32 < big ? 32 : 0;
+}
+
 int gemm_launch(const GemmArgs &a, int64_t ntiles, hipStream_t st) {
     using namespace gm;
     if (a.k <= 0 || a.k % KC != 0 || a.nr <= 0 || a.ldy < a.nr) return -1;
@@ -253,6 +477,15 @@ int gemm_launch(const GemmArgs &a, int64_t ntiles, hipStream_t st) {
     if (ny <= 0) return 0;
     // 16-byte output (and residual) accesses where every row group of 4 starts 16-byte aligned
     const int vec4 = a.ldy % 4 == 0 && (uintptr_t)a.y % 16 == 0 && (!a.res || (a.ldr % 4 == 0 && (uintptr_t)a.res % 16 == 0));
+    // grouped tiles stay with the large tile: a prompt of 61 tokens streams its experts at 5 TB/s with it (a
+    // whole prefill 11.1 ms; their tiles by single waves of 16 or 32: 13.8, 12.7)
+    const int ts = a.tiles ? 0 : small_tile(a.nr, a.nt);
+    if (ts > 0) {
+        const dim3 g((unsigned)((a.nr + ts - 1) / ts), (unsigned)((a.nt + ts - 1) / ts));
+        if (ts == 16) hipLaunchKernelGGL(gemm_q8_small_kernel<16>, g, dim3(64), 0, st, a, vec4);
+        else hipLaunchKernelGGL(gemm_q8_small_kernel<32>, g, dim3(64), 0, st, a, vec4);
+        return hipGetLastError() == hipSuccess ? 0 : -2;
+    }
     hipLaunchKernelGGL(gemm_q8_kernel, dim3((unsigned)((a.nr + BM - 1) / BM), (unsigned)ny), dim3(NT), 0, st, a, vec4);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
