@@ -120,12 +120,25 @@ def exported_symbols():
 
 
 def _p(t):
-    return C.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
+
+
+_raw_stream = None
 
 
 def _stream():
-    import torch
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """handle of the current device's current stream: the raw getter where torch has it (the Stream object
+    of torch.cuda.current_stream() costs more than the rest of a small call)"""
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
+        torch.cuda.current_stream()   # initialises the device
+        raw, dev = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
+        if raw is not None and dev is not None:
+            _raw_stream = lambda: raw(dev())  # noqa: E731
+        else:
+            _raw_stream = lambda: torch.cuda.current_stream().cuda_stream  # noqa: E731
+    return _raw_stream()
 
 
 def check(rc, what):
