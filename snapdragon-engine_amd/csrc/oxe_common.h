@@ -49,6 +49,7 @@ OXE_DEV int shfl_xor_i(int v, int m) { return __shfl_xor(v, m, 64); }
 // quad_perm gives ^ 1 and ^ 2 directly.
 constexpr int DPP_XOR1 = 0xB1;   // quad_perm [1, 0, 3, 2]
 constexpr int DPP_XOR2 = 0x4E;   // quad_perm [2, 3, 0, 1]
+constexpr int DPP_HALF_MIRROR = 0x141;   // lane i of each 8 takes lane 7 - i: ^ 4 once the quads are uniform
 constexpr int DPP_ROR1 = 0x121, DPP_ROR2 = 0x122, DPP_ROR4 = 0x124, DPP_ROR8 = 0x128;
 template <int CTRL>
 OXE_DEV int dpp_i(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false); }
