@@ -251,7 +251,7 @@ OXE_DEV float chain(float acc, const uint8_t *wb, float dx, const int *r0, const
 
 // ---- the lane GEMV --------------------------------------------------------------------------------
 // s[l * nr + r] = W[r] . y[l]; w: nr rows of nb blocks (row bytes a multiple of 4, w 16-byte
-// aligned); y: NL lanes of nb q8_K blocks. One wave per workgroup, persistent over groups of 4 rows
+// aligned); y: NL lanes of nb q8_K blocks. Waves persistent over groups of 4 rows, NW of them to a workgroup
 // (16 threads per row). Per group: the 4 rows' bytes (contiguous) go to LDS with 16-byte loads, the
 // first PF x 1 KiB of them held in registers, two groups ahead (buffers a and b, alternating); then
 // per chunk of up to 8 blocks thread (row ri, unit u) forms half block u % 2 of block u / 2 for
@@ -320,26 +320,42 @@ OXE_DEV SegRef seg_ref(const KqSegs &S, int64_t g) {
 
 // one group of 4 rows (g may be past the end: then nothing is written): its prefetched bytes (pf)
 // and the rest to LDS, pf refilled with group g_next, then the units and the chains
-template <int TY, int NL, int PF>
+// LDS accesses of this wave before it come before those after it (wave-private regions: no barrier)
+OXE_DEV void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+template <int NW>
+OXE_DEV void group_sync() {
+    if (NW == 1) __syncthreads();   // one wave: a wait for its LDS accesses (the fence alone measured 5-10 % slower)
+    else wave_fence();
+}
+// LDS of one wave: a group's rows and its units' integers
+__host__ __device__ inline int vl_wave_lds(int bb, int rr, int nb, int nl) {
+    return align16(GR * nb * bb) + align16(64 * ((nl * rr) | 1) * 4);
+}
+
+template <int TY, int NL, int PF, int NW>
 OXE_DEV void vl_group(u32x4 (&pf)[PF], int64_t g, int64_t g_next, const KqSegs &S, int nb, float *__restrict__ s,
                       const KqEpi &epi, uint8_t *wl, const uint32_t *yh, const float *yd, int *res) {
     constexpr int BB = BT<TY>::B;
     constexpr int RES = BT<TY>::R;
     constexpr int RS = (NL * RES) | 1;   // odd per-thread stride: no bank conflicts between threads
     const int row_bytes = nb * BB, ls = y_lane_words(nb);
-    const int t = threadIdx.x, ri = t >> 4, u = t & 15;
+    const int t = NW == 1 ? threadIdx.x : threadIdx.x & 63, ri = t >> 4, u = t & 15;
     const int64_t ngroups = S.ngroups;
     const bool gin = g < ngroups;
     const SegRef sg = seg_ref(S, gin ? g : ngroups - 1);   // the group whose bytes pf holds
     const int64_t nr = sg.nr;
     const int sp = (int)(min((int64_t)GR, nr - sg.gl * GR) * row_bytes), n16 = sp / 16;
     const u32x4 *src = (const u32x4 *)(sg.w + sg.gl * GR * row_bytes);
-    __syncthreads();   // the previous group's LDS reads are done
+    group_sync<NW>();   // the previous group's LDS reads come first
 #pragma unroll
     for (int j = 0; j < PF; j++) ((u32x4 *)wl)[min(t + 64 * j, n16 - 1)] = pf[j];   // clamped: same bytes
     for (int i = t + 64 * PF; i < n16; i += 64) ((u32x4 *)wl)[i] = src[i];
     for (int i = n16 * 4 + t; i < sp / 4; i += 64) ((uint32_t *)wl)[i] = ((const uint32_t *)src)[i];   // tail
-    __syncthreads();
+    group_sync<NW>();
     {
         const SegRef sn = seg_ref(S, g_next < ngroups ? g_next : ngroups - 1);
         pf_load(pf, sn.w, sn.gl, sn.nr, row_bytes, t);   // in flight meanwhile
@@ -352,14 +368,14 @@ OXE_DEV void vl_group(u32x4 (&pf)[PF], int64_t g, int64_t g_next, const KqSegs &
         const int bi = b0 + (u >> 1);
         if ((u >> 1) < kc && live)
             unit<TY, NL>(wl + ri * row_bytes + bi * BB, YView{yh + (2 * bi + (u & 1)) * YH, ls}, u & 1, res + t * RS);
-        __syncthreads();
+        group_sync<NW>();
         if (u < NL && live)
             for (int b = 0; b < kc; b++) {
                 const int *r0 = res + (ri * 16 + 2 * b) * RS + u * RES;
                 const int *r1 = res + (ri * 16 + 2 * b + 1) * RS + u * RES;
                 acc = chain<TY>(acc, wl + ri * row_bytes + (b0 + b) * BB, yd[u * nb + b0 + b], r0, r1);
             }
-        __syncthreads();
+        group_sync<NW>();
     }
     if (u < NL && live) {
         if (!epi.ctl) {
@@ -373,51 +389,53 @@ OXE_DEV void vl_group(u32x4 (&pf)[PF], int64_t g, int64_t g_next, const KqSegs &
     }
 }
 
-template <int TY, int NL, int PF>
-__global__ __launch_bounds__(64) void vl_gemv_kernel(KqSegs S, int nb, const uint8_t *__restrict__ y,
-                                                     float *__restrict__ s, KqEpi epi) {
+template <int TY, int NL, int PF, int NW>
+__global__ __launch_bounds__(64 * NW) void vl_gemv_kernel(KqSegs S, int nb, const uint8_t *__restrict__ y,
+                                                          float *__restrict__ s, KqEpi epi) {
     constexpr int BB = BT<TY>::B;
     extern __shared__ __align__(16) uint8_t lds[];
     const int row_bytes = nb * BB;
-    uint8_t *wl = lds;                                                   // [GR][row_bytes]
-    uint32_t *yh = (uint32_t *)(lds + align16(GR * row_bytes));         // [NL][nb][2][YH]
+    const int t = NW == 1 ? threadIdx.x : threadIdx.x & 63, w = NW == 1 ? 0 : threadIdx.x >> 6;
+    // the lanes' activations, shared; then per wave a group's rows and the units' integers
+    const int ys = align16(NL * nb * (2 * YH + 1) * 4);
+    uint8_t *wl = lds + (NW == 1 ? 0 : ys + (size_t)w * vl_wave_lds(BB, BT<TY>::R, nb, NL));   // [GR][row_bytes]
+    uint32_t *yh = (uint32_t *)(lds + (NW == 1 ? align16(GR * row_bytes) : 0));   // [NL][nb][2][YH]
     float *yd = (float *)(yh + NL * y_lane_words(nb));                   // [NL][nb]
-    int *res = (int *)((uint8_t *)yh + align16(NL * nb * (2 * YH + 1) * 4));   // [64][(NL * R) | 1]
-    const int t = threadIdx.x;
-    const int64_t ngroups = S.ngroups, G = gridDim.x;
+    int *res = (int *)(wl + align16(GR * row_bytes) + (NW == 1 ? ys : 0));   // [64][(NL * R) | 1]
+    const int64_t ngroups = S.ngroups, G = (int64_t)gridDim.x * NW, g0 = (int64_t)blockIdx.x * NW + w;
     // the lanes' q8_K blocks (lane l block b is block l nb + b) repacked into halves and scales
-    for (int i = t; i < NL * nb * 2 * 36; i += 64) {
+    for (int i = threadIdx.x; i < NL * nb * 2 * 36; i += 64 * NW) {
         const int wd = i % 36, hb = i / 36, h = hb & 1;
         const uint32_t *src = (const uint32_t *)(y + (int64_t)(hb >> 1) * Q8K_BYTES);
         yh[hb * YH + wd] = wd < 32 ? src[1 + 32 * h + wd] : src[65 + 4 * h + (wd - 32)];
     }
-    for (int i = t; i < NL * nb; i += 64) yd[i] = *(const float *)(y + (int64_t)i * Q8K_BYTES);
+    for (int i = threadIdx.x; i < NL * nb; i += 64 * NW) yd[i] = *(const float *)(y + (int64_t)i * Q8K_BYTES);
     // two register buffers (fixed indices only: they stay in registers), groups g and g + G in
     // flight from the start; the scheduling barrier keeps buffer a's loads ahead of b's, so the
     // first LDS stores wait for a's only
     u32x4 pa[PF], pb[PF];
-    if ((int64_t)blockIdx.x >= ngroups) return;
     {
-        const SegRef sa = seg_ref(S, blockIdx.x), sb = seg_ref(S, min((int64_t)blockIdx.x + G, ngroups - 1));
+        const SegRef sa = seg_ref(S, min(g0, ngroups - 1)), sb = seg_ref(S, min(g0 + G, ngroups - 1));
         pf_load(pa, sa.w, sa.gl, sa.nr, row_bytes, t);
         __builtin_amdgcn_sched_barrier(0);
         pf_load(pb, sb.w, sb.gl, sb.nr, row_bytes, t);
     }
-    for (int64_t g = blockIdx.x; g < ngroups; g += 2 * G) {
-        vl_group<TY, NL, PF>(pa, g, g + 2 * G, S, nb, s, epi, wl, yh, yd, res);
-        vl_group<TY, NL, PF>(pb, g + G, g + 3 * G, S, nb, s, epi, wl, yh, yd, res);
+    if (NW > 1) __syncthreads();
+    for (int64_t g = g0; g < ngroups; g += 2 * G) {
+        vl_group<TY, NL, PF, NW>(pa, g, g + 2 * G, S, nb, s, epi, wl, yh, yd, res);
+        vl_group<TY, NL, PF, NW>(pb, g + G, g + 3 * G, S, nb, s, epi, wl, yh, yd, res);
     }
 }
 
-size_t vl_gemv_lds(int bb, int rr, int nb, int nl) {
-    return (size_t)align16(GR * nb * bb) + (size_t)align16(nl * nb * (2 * YH + 1) * 4) + (size_t)64 * ((nl * rr) | 1) * 4;
+size_t vl_gemv_lds(int bb, int rr, int nb, int nl, int nw) {
+    return (size_t)align16(nl * nb * (2 * YH + 1) * 4) + (size_t)nw * vl_wave_lds(bb, rr, nb, nl);
 }
 
 constexpr int KQ_MAX_DEV = 64;
-template <int TY, int NL, int PF>
-int vl_gemv_launch_pf(const KqSegs &S, int nb, const uint8_t *y, float *s, hipStream_t st, const KqEpi &epi) {
+template <int TY, int NL, int PF, int NW>
+int vl_gemv_launch_nw(const KqSegs &S, int nb, const uint8_t *y, float *s, hipStream_t st, const KqEpi &epi) {
     constexpr int BB = BT<TY>::B;
-    const size_t lds = vl_gemv_lds(BB, BT<TY>::R, nb, NL);
+    const size_t lds = vl_gemv_lds(BB, BT<TY>::R, nb, NL, NW);
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= KQ_MAX_DEV) return -2;
     // per instantiation and device: the dynamic LDS the kernel is configured for (above 64 KiB it
@@ -436,7 +454,7 @@ int vl_gemv_launch_pf(const KqSegs &S, int nb, const uint8_t *y, float *s, hipSt
         std::lock_guard<std::mutex> lk(mu);
         Cache &cc = cache[dev];
         if (lds > cc.configured) {
-            if (hipFuncSetAttribute((const void *)vl_gemv_kernel<TY, NL, PF>, hipFuncAttributeMaxDynamicSharedMemorySize,
+            if (hipFuncSetAttribute((const void *)vl_gemv_kernel<TY, NL, PF, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)lds) != hipSuccess)
                 return -2;
             cc.configured = lds;
@@ -454,7 +472,7 @@ int vl_gemv_launch_pf(const KqSegs &S, int nb, const uint8_t *y, float *s, hipSt
             // last waves to start after others finish, one below them leaves SIMDs short of a wave
             // (measured on the Q6_K LM head, 12 resident per CU: 11 per CU 131 us, 13 per CU 116 us,
             // 12 per CU 92.5 us)
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, vl_gemv_kernel<TY, NL, PF>, 64, lds) != hipSuccess ||
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, vl_gemv_kernel<TY, NL, PF, NW>, 64 * NW, lds) != hipSuccess ||
                 occ < 1)
                 occ = (int)std::max<size_t>(1, (160 * 1024) / lds);
             if (slot >= 0) {
@@ -463,19 +481,34 @@ int vl_gemv_launch_pf(const KqSegs &S, int nb, const uint8_t *y, float *s, hipSt
             }
         }
     }
-    const int per_cu = std::min(16, occ);
-    const int64_t grid = std::min<int64_t>(S.ngroups, (int64_t)ncu * per_cu);
-    hipLaunchKernelGGL((vl_gemv_kernel<TY, NL, PF>), dim3((unsigned)grid), dim3(64), lds, st, S, nb, y, s, epi);
+    const int64_t grid = std::min<int64_t>((S.ngroups + NW - 1) / NW, (int64_t)ncu * std::max(1, std::min(16 / NW, occ)));
+    hipLaunchKernelGGL((vl_gemv_kernel<TY, NL, PF, NW>), dim3((unsigned)grid), dim3(64 * NW), lds, st, S, nb, y, s, epi);
     return hipGetLastError() == hipSuccess ? 1 : -2;
 }
+// Four waves share the lanes' activations in LDS where staging them is what a workgroup spends its time on: at
+// least two lanes of rows of 2048 (Q3_K, whose waves need the most registers: 24 blocks in all; Q6_K also one lane of 3072).
+// Measured, one wave against four (us): Q4_K 8192 x 2048 2 lanes 11.4 / 9.4, 4 lanes 15.1 / 10.7, 100000 x 4096 4 lanes
+// 160 / 106; Q6_K 100000 x 3072 2 lanes 113 / 68; but one lane 700 x 2048 Q4_K 6.2 / 7.3, 100000 x 1024 24.3 / 27.1
+template <int TY, int NL, int PF>
+int vl_gemv_launch_pf(const KqSegs &S, int nb, const uint8_t *y, float *s, hipStream_t st, const KqEpi &epi) {
+    if constexpr (PF >= 4 && (NL >= 2 || TY == 6)) {
+        const bool wide = NL >= 2 ? nb >= 8 && (TY != 3 || NL * nb >= 24) : nb >= 12;
+        if (wide && vl_gemv_lds(BT<TY>::B, BT<TY>::R, nb, NL, 4) <= 80 * 1024)
+            return vl_gemv_launch_nw<TY, NL, PF, 4>(S, nb, y, s, st, epi);
+    }
+    return vl_gemv_launch_nw<TY, NL, PF, 1>(S, nb, y, s, st, epi);
+}
 
-// registers per prefetch buffer: the smallest of 2, 4, 8 KiB-per-wave steps that holds a whole group
+// registers per prefetch buffer: the smallest of 2, 4, a row-of-2048 group's, 8 KiB per wave that holds a whole group
 // (the rest of a larger group is copied to LDS directly)
 template <int TY, int NL>
 int vl_gemv_launch(const KqSegs &S, int nb, const uint8_t *y, float *s, hipStream_t st, const KqEpi &epi) {
     const int n16 = GR * nb * BT<TY>::B / 16;
     if (n16 <= 128) return vl_gemv_launch_pf<TY, NL, 2>(S, nb, y, s, st, epi);
     if (n16 <= 256) return vl_gemv_launch_pf<TY, NL, 4>(S, nb, y, s, st, epi);
+    constexpr int P = (GR * 8 * BT<TY>::B / 16 + 63) / 64;   // a group of rows of 2048
+    if constexpr (P > 4)
+        if (n16 <= 64 * P) return vl_gemv_launch_pf<TY, NL, P>(S, nb, y, s, st, epi);
     return vl_gemv_launch_pf<TY, NL, 8>(S, nb, y, s, st, epi);
 }
 
