@@ -17,14 +17,15 @@
 // The block scale products d_w * d_x are rank-1 f32 matrix products (nothing added to each product,
 // so each is the correctly rounded one).
 //
-// Workgroup: NW waves of 32 weight rows x up to 64 tokens (two 32 x 32 tiles). A wave unpacks its own
-// rows' blocks in registers, straight from global memory (no other wave reads them, so LDS would only
-// add a round trip), one block ahead. The tokens' codes go through LDS, one block per stage, double
-// buffered, by direct global-to-LDS loads; 128-byte code rows with their 16-byte chunks XOR-swizzled by
-// f(r) = (r & 7) ^ ((r >> 3) & 1), as the Q8_0 GEMM's.
+// Workgroup: NW waves of 32 weight rows x up to 64 tokens (two 32 x 32 tiles). A wave stages its own rows' blocks
+// through LDS of its own (no barrier: no other wave reads them), loaded as whole lines one block ahead; unpacked straight
+// from global memory, 32 rows apart per load, a single-wave workgroup ([2048 x 4096], 701 tokens, Q4_K) took 83 us against
+// 55. The tokens' codes go through LDS shared by the waves, 256 bytes a row per stage, double buffered, by direct
+// global-to-LDS loads; 128-byte code rows with their 16-byte chunks XOR-swizzled by f(r) = (r & 7) ^ ((r >> 3) & 1), as the
+// Q8_0 GEMM's. Bound by the VALU (unpacking, and the chain) at two waves per SIMD.
 //
-// Measured, [12288 x 2048] over 2048 tokens with its quantisation: Q3_K 152 us, Q4_K 223, Q5_K 292, Q6_K 240.
-// A 701-token prompt through 8 layers of the Ornith file's types: 421 ms as decode runs of two positions, 5.3 ms.
+// Measured, [12288 x 2048] over 2048 tokens with its quantisation: Q3_K 147 us, Q4_K 238, Q5_K 321, Q6_K 231.
+// A 701-token prompt through 8 layers of the Ornith file's types: 419 ms as decode runs of two positions, 5.1 ms.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -68,86 +69,61 @@ OXE_DEV h2 byte_pair(uint32_t w) {
     const uint32_t u = __builtin_amdgcn_perm(0x64646464u, w, 0x04000400u + 0x00010001u * I);
     return as_h2(u) - h2{(_Float16)1024.0f, (_Float16)1024.0f};
 }
-// N dwords at byte address p of any 2-byte alignment: the N + 1 dwords around them, cut when used
-template <int N>
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// 16 bytes (and the two after them) at LDS address p + sh, p a multiple of 16, sh 0 or 2
 struct Run {
-    uint32_t w[N + 1];
-    uint32_t sh;
+    u32x4 w;
+    uint32_t x;
     OXE_DEV void load(const uint8_t *p) {
-        sh = (uint32_t)(uintptr_t)p & 3u;
-        const uint32_t *a = (const uint32_t *)(p - sh);
-#pragma unroll
-        for (int i = 0; i <= N; i++) w[i] = a[i];
+        w = *(const u32x4 *)p;
+        x = *(const uint32_t *)(p + 16);
     }
-    OXE_DEV uint32_t get(int i) const { return __builtin_amdgcn_alignbyte(w[i + 1], w[i], sh); }
+    OXE_DEV uint32_t get(int i, int sh) const { return __builtin_amdgcn_alignbyte(i < 3 ? w[i + 1] : x, w[i], sh); }
 };
 
-// ---- one lane's share of a block: row lane & 31, half hf = lane >> 5 of every 32-weight sub-block ---
-// Q4_K / Q5_K: bytes 16 hf .. 16 hf + 15 of each 64-weight step's 32 nibble bytes
-template <int TY> struct Raw;
-template <> struct Raw<4> {
-    uint4 hdr, qs[4];
-    OXE_DEV void load(const uint8_t *b, int hf) {
-        hdr = *(const uint4 *)b;
-#pragma unroll
-        for (int g = 0; g < 4; g++) qs[g] = *(const uint4 *)(b + 16 + 32 * g + 16 * hf);
-    }
-};
-template <> struct Raw<5> {
-    uint4 hdr, qs[4], qh;
-    OXE_DEV void load(const uint8_t *b, int hf) {
-        hdr = *(const uint4 *)b;
-        qh = *(const uint4 *)(b + 16 + 16 * hf);
-#pragma unroll
-        for (int g = 0; g < 4; g++) qs[g] = *(const uint4 *)(b + 48 + 32 * g + 16 * hf);
-    }
-};
-// Q3_K: bytes 16 hf .. of the high-bit mask and of each 128-weight half's codes; scales and d
-template <> struct Raw<3> {
-    Run<4> hm, qs[2];
-    uint32_t sd[4], sh;   // the dwords around bytes 96..109
+// A block's bytes as a wave stages them: 32 rows, CH chunks of 16 bytes each, STRIDE bytes apart in LDS (8 consecutive
+// rows' 16-byte reads fall on distinct banks). Q3_K / Q6_K blocks (110 / 210 bytes) of odd index start 2 bytes past a
+// dword (rows hold an even number of blocks): they are staged from the dword before, and read with that shift.
+template <int TY> struct Geo;
+template <> struct Geo<3> { static constexpr int BB = 110, CH = 7, STRIDE = 112; };
+template <> struct Geo<4> { static constexpr int BB = 144, CH = 9, STRIDE = 144; };
+template <> struct Geo<5> { static constexpr int BB = 176, CH = 11, STRIDE = 176; };
+template <> struct Geo<6> { static constexpr int BB = 210, CH = 14, STRIDE = 240; };
+
+// ---- one lane's share of a staged block: row lane & 31, half hf = lane >> 5 of every 32-weight sub-block -------
+// Q3_K: bytes 16 hf .. of the high-bit mask and of each 128-weight half's codes; Q6_K: of each half's low and high
+// code bits
+struct Raw3 {
+    Run hm, qs[2];
     OXE_DEV void load(const uint8_t *b, int hf) {
         hm.load(b + 16 * hf);
 #pragma unroll
         for (int n = 0; n < 2; n++) qs[n].load(b + 32 + 32 * n + 16 * hf);
-        sh = (uint32_t)(uintptr_t)b & 3u;
-        const uint32_t *a = (const uint32_t *)(b + 96 - sh);
-#pragma unroll
-        for (int i = 0; i < 4; i++) sd[i] = a[i];
     }
 };
-template <> struct Raw<6> {
-    Run<4> ql[2][2], qh[2];
-    uint32_t sd[5], sh;   // the dwords around bytes 192..209
-    OXE_DEV void load(const uint8_t *b, int hf) {
-#pragma unroll
-        for (int n = 0; n < 2; n++) {
-            ql[n][0].load(b + 64 * n + 16 * hf);
-            ql[n][1].load(b + 64 * n + 32 + 16 * hf);
-            qh[n].load(b + 128 + 32 * n + 16 * hf);
-        }
-        sh = (uint32_t)(uintptr_t)b & 3u;
-        const uint32_t *a = (const uint32_t *)(b + 192 - sh);
-#pragma unroll
-        for (int i = 0; i < 5; i++) sd[i] = a[i];
+struct Raw6 {
+    Run ql[2], qh;
+    OXE_DEV void load(const uint8_t *b, int hf, int n) {
+        ql[0].load(b + 64 * n + 16 * hf);
+        ql[1].load(b + 64 * n + 32 + 16 * hf);
+        qh.load(b + 128 + 32 * n + 16 * hf);
     }
 };
-
-OXE_DEV uint32_t sel4(const uint4 &v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
 
 // the f16 fragments of one 64-weight step: lo / hi 32 weights (p), matrix product m of 16
+// (qs: the lane's 16 nibble bytes of the step; qh: Q5_K's high-bit bytes)
 template <int TY>
-OXE_DEV void step_frags(const Raw<TY> &r, int g, h2 s_lo, h2 s_hi, uint32_t (&lo)[2][4], uint32_t (&hi)[2][4]) {
+OXE_DEV void step_frags(u32x4 qs, u32x4 qh, int g, h2 s_lo, h2 s_hi, uint32_t (&lo)[2][4], uint32_t (&hi)[2][4]) {
     const h2 k1024 = h2{(_Float16)-1024.0f, (_Float16)-1024.0f};
     const h2 c_lo = s_lo * k1024, c_hi = s_hi * k1024;   // exact: at most 63 * 2^10
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const uint32_t w = sel4(r.qs[g], i);
+        const uint32_t w = qs[i];
         // pairs (code 0, code 2) and (code 1, code 3) of the dword's four bytes
         uint32_t l0 = (w & 0x000f000fu) | 0x64006400u, l1 = ((w >> 8) & 0x000f000fu) | 0x64006400u;
         uint32_t h0 = ((w >> 4) & 0x000f000fu) | 0x64006400u, h1 = ((w >> 12) & 0x000f000fu) | 0x64006400u;
         if constexpr (TY == 5) {
-            const uint32_t q = sel4(r.qh, i);
+            const uint32_t q = qh[i];
             const uint32_t bl = (q >> (2 * g)) & 0x01010101u, bh = (q >> (2 * g + 1)) & 0x01010101u;
             l0 |= (bl & 0x00010001u) << 4;
             l1 |= (bl >> 4) & 0x00100010u;
@@ -164,26 +140,26 @@ OXE_DEV void step_frags(const Raw<TY> &r, int g, h2 s_lo, h2 s_hi, uint32_t (&lo
 
 // Q3_K, sub-block j of half n: the 16 codes' products with s = 32 - raw scale, by byte lookup:
 // (code - 4) * s for code 0..7 in two dwords
-OXE_DEV void q3_frag(const Raw<3> &r, int n, int j, int s, uint32_t (&f)[4]) {
+OXE_DEV void q3_frag(const Raw3 &r, int sh, int n, int j, int s, uint32_t (&f)[4]) {
     const uint32_t s1 = (uint32_t)s & 255u, s2 = (uint32_t)(2 * s) & 255u, s3 = (uint32_t)(3 * s) & 255u;
     const uint32_t n1 = (uint32_t)-s & 255u, n2 = (uint32_t)(-2 * s) & 255u, n3 = (uint32_t)(-3 * s) & 255u;
     const uint32_t n4 = (uint32_t)(-4 * s) & 255u;
     const uint32_t thi = s1 << 8 | s2 << 16 | s3 << 24, tlo = n4 | n3 << 8 | n2 << 16 | n1 << 24;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const uint32_t c = ((r.qs[n].get(i) >> (2 * j)) & 0x03030303u) | (((r.hm.get(i) >> (4 * n + j)) & 0x01010101u) << 2);
+        const uint32_t c = ((r.qs[n].get(i, sh) >> (2 * j)) & 0x03030303u) | (((r.hm.get(i, sh) >> (4 * n + j)) & 0x01010101u) << 2);
         f[i] = __builtin_amdgcn_perm(thi, tlo, c);
     }
 }
 
 typedef short s2v __attribute__((ext_vector_type(2)));
 // Q6_K, sub-block q of half n: s * (code - 32) = 64 h + l of the 16 codes
-OXE_DEV void q6_frag(const Raw<6> &r, int n, int q, int s, uint32_t (&fh)[4], uint32_t (&fl)[4]) {
+OXE_DEV void q6_frag(const Raw6 &r, int sh, int q, int s, uint32_t (&fh)[4], uint32_t (&fl)[4]) {
     const s2v sv = {(short)s, (short)s}, off = {(short)(-32 * s), (short)(-32 * s)};
     const s2v six = {6, 6};
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const uint32_t a = r.ql[n][q & 1].get(i) >> (q >= 2 ? 4 : 0), b = r.qh[n].get(i);
+        const uint32_t a = r.ql[q & 1].get(i, sh) >> (q >= 2 ? 4 : 0), b = r.qh.get(i, sh);
         const uint32_t c = (a & 0x0f0f0f0fu) | (((b >> (2 * q)) & 0x03030303u) << 4);
         const s2v e = __builtin_bit_cast(s2v, c & 0x00ff00ffu), o = __builtin_bit_cast(s2v, (c >> 8) & 0x00ff00ffu);
         const s2v ve = e * sv + off, vo = o * sv + off;
@@ -196,16 +172,25 @@ OXE_DEV void q6_frag(const Raw<6> &r, int n, int q, int s, uint32_t (&fh)[4], ui
 
 constexpr int BN = 64;   // tokens per workgroup
 
+// LDS accesses of this wave before it come before those after it (wave-private rows: no barrier)
+OXE_DEV void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // chunk swizzle of a 128-byte code row
 OXE_DEV int swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
 template <int TY, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void kq_gemm_kernel(KqGemmArgs a) {
     constexpr bool F16 = TY == 4 || TY == 5;
+    using G = Geo<TY>;
     constexpr int XB = F16 ? 512 : 256;   // code bytes of a token and block
-    constexpr int NU = XB / 128;          // 128-byte units
-    constexpr int BB = TY == 3 ? 110 : TY == 4 ? 144 : TY == 5 ? 176 : 210;
-    __shared__ __align__(16) uint8_t sx[2][NU * BN * 128];
+    constexpr int SPB = XB / 256;         // token stages per block, of two 128-byte units
+    constexpr int NLD = (32 * G::CH + 63) / 64;   // 16-byte weight loads per lane and block
+    __shared__ __align__(16) uint8_t sx[2][2 * BN * 128];
+    __shared__ __align__(16) uint8_t sw[NW][32 * G::STRIDE];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, fr = lane & 31, hf = lane >> 5;
     const int nb = a.nb;
     // the row tile's segment (fixed indices: the table stays in the kernel arguments)
@@ -232,8 +217,16 @@ __global__ __launch_bounds__(64 * NW, 2) void kq_gemm_kernel(KqGemmArgs a) {
     if (pn <= 0) return;   // uniform
     const int64_t r0 = (int64_t)tile * (32 * NW) + 32 * w;
     const bool wave_on = r0 < sg.nr;   // wave-uniform
-    const int64_t wrow = r0 + fr < sg.nr ? r0 + fr : sg.nr - 1;
-    const uint8_t *wr = wb + wrow * (int64_t)nb * BB;
+    // weight loads: lane's chunk i = lane + 64 j of the wave's 32 rows x CH chunks (past the rows: the last row's)
+    uint32_t wofs[NLD];
+    int wdst[NLD];
+#pragma unroll
+    for (int j = 0; j < NLD; j++) {
+        const int i = lane + 64 * j < 32 * G::CH ? lane + 64 * j : 32 * G::CH - 1, r = i / G::CH, c = i % G::CH;
+        const int64_t row = r0 + r < sg.nr ? r0 + r : sg.nr - 1;
+        wofs[j] = (uint32_t)(row * (int64_t)nb * G::BB + 16 * c);
+        wdst[j] = r * G::STRIDE + 16 * c;
+    }
     // activation row of token slot i of the tile (past the tile: its first token, never stored)
     auto xrow = [&](int i) -> int64_t {
         const int64_t p = p0 + (i < pn ? i : 0);
@@ -250,13 +243,13 @@ __global__ __launch_bounds__(64 * NW, 2) void kq_gemm_kernel(KqGemmArgs a) {
             xofs[k] = (uint32_t)(xrow(row) * (int64_t)nb * XB + 16 * ((lane & 7) ^ swz(row)));
         }
         const uint8_t *xc = F16 ? (const uint8_t *)a.x.c16 : (const uint8_t *)a.x.c8;
-        auto fetch = [&](int buf, int b) {
+        auto fetch = [&](int buf, int st) {   // stage st: code bytes 256 st .. of every token row
 #pragma unroll
             for (int k = 0; k < RPW; k++)
                 if (w * RPW + k < RG) {
 #pragma unroll
-                    for (int u = 0; u < NU; u++)
-                        to_lds16(xc + (xofs[k] + (uint32_t)(b * XB + 128 * u)), &sx[buf][(u * BN + 8 * (w * RPW + k)) * 128]);
+                    for (int u = 0; u < 2; u++)
+                        to_lds16(xc + (xofs[k] + (uint32_t)(st * 256 + 128 * u)), &sx[buf][(u * BN + 8 * (w * RPW + k)) * 128]);
                 }
         };
         // block scale of token `lane` (both tiles in one rank-1 product) and, Q4_K / Q5_K, the sums of
@@ -266,17 +259,27 @@ __global__ __launch_bounds__(64 * NW, 2) void kq_gemm_kernel(KqGemmArgs a) {
         const uint16_t *bsp[NJ];
 #pragma unroll
         for (int j = 0; j < NJ; j++) bsp[j] = F16 ? a.x.bs + xrow(32 * j + fr) * (int64_t)nb * 16 + 8 * hf : nullptr;
-        Raw<TY> raw;
+        u32x4 stg[NLD];
         float dx = 0.0f;
         i32x4 bs[NJ];
         auto wload = [&](int b) {
-            raw.load(wr + (int64_t)b * BB, hf);
+            const uint8_t *p = wb + (b * G::BB - (F16 ? 0 : 2 * (b & 1)));
+#pragma unroll
+            for (int j = 0; j < NLD; j++) __builtin_memcpy(&stg[j], __builtin_assume_aligned(p + wofs[j], F16 ? 16 : 4), 16);
             dx = xdp[b];
             if constexpr (F16) {
 #pragma unroll
                 for (int j = 0; j < NJ; j++) bs[j] = *(const i32x4 *)(bsp[j] + 16 * b);
             }
         };
+        // the staged block to this wave's LDS rows: its reads of the block before come first, those of this one after
+        auto wput = [&]() {
+            wave_fence();
+#pragma unroll
+            for (int j = 0; j < NLD; j++) *(u32x4 *)&sw[w][wdst[j]] = stg[j];
+            wave_fence();
+        };
+        const uint8_t *wl = &sw[w][fr * G::STRIDE];   // this lane's row
         float acc[NJ][16];
 #pragma unroll
         for (int j = 0; j < NJ; j++)
@@ -287,18 +290,34 @@ __global__ __launch_bounds__(64 * NW, 2) void kq_gemm_kernel(KqGemmArgs a) {
         auto frag = [&](int buf, int u, int c, int j) {
             return *(const i32x4 *)&sx[buf][(u * BN + 32 * j + fr) * 128 + 16 * (c ^ swz(fr))];
         };
-        auto compute = [&](int buf, const Raw<TY> &r, float dxb, const i32x4 (&bsb)[NJ]) {
-            if (!wave_on) return;
+        auto stage_sync = [&]() {
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+        };
+        const int ns = nb * SPB;
+        fetch(0, 0);
+        wload(0);
+        for (int b = 0; b < nb; b++) {
+            stage_sync();   // the stage's codes in LDS, every wave done with the other buffer
+            const float dxb = dx;
+            i32x4 bsb[NJ];
+#pragma unroll
+            for (int j = 0; j < NJ; j++) bsb[j] = bs[j];
+            if (SPB * b + 1 < ns) fetch((SPB * b + 1) & 1, SPB * b + 1);
+            wput();
+            if (b + 1 < nb) wload(b + 1);
             if constexpr (F16) {
-                const float dw = h2f((uint16_t)r.hdr.x), dm = h2f((uint16_t)(r.hdr.x >> 16));
+                const u32x4 hdr = *(const u32x4 *)wl;
+                u32x4 qh = {};
+                if constexpr (TY == 5) qh = *(const u32x4 *)(wl + 16 + 16 * hf);
+                const float dw = h2f((uint16_t)hdr[0]), dm = h2f((uint16_t)(hdr[0] >> 16));
                 // the eight 6-bit scales and mins, four bytes a dword (get_scale_min_k4)
-                const uint32_t s0 = r.hdr.y, s1 = r.hdr.z, s2 = r.hdr.w;
+                const uint32_t s0 = hdr[1], s1 = hdr[2], s2 = hdr[3];
                 const uint32_t sc[2] = {s0 & 0x3f3f3f3fu, (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u)};
                 const uint32_t mn = hf ? ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u) : s1 & 0x3f3f3f3fu;
                 const f32x32 ds = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, dxb, zero32, 0, 0, 0);
                 uint32_t mf[4] = {as_u(byte_pair<0>(mn)), as_u(byte_pair<1>(mn)), as_u(byte_pair<2>(mn)), as_u(byte_pair<3>(mn))};
-                // acc -= (sum of mins * code sums) * (dmin * d_x); the scale products are formed again for
-                // each use rather than held in 32 registers through the block
+                // acc -= (sum of mins * code sums) * (dmin * d_x)
                 auto mins = [&](const uint32_t (&f)[4]) {
                     const f32x32 ms = __builtin_amdgcn_mfma_f32_32x32x1f32(dm, dxb, zero32, 0, 0, 0);
 #pragma unroll
@@ -311,124 +330,134 @@ __global__ __launch_bounds__(64 * NW, 2) void kq_gemm_kernel(KqGemmArgs a) {
                         }
                     }
                 };
-                auto step = [&](auto gc) {
+                auto step = [&](int buf, auto gc) {
                     constexpr int g = decltype(gc)::value;
                     uint32_t lo[2][4], hi[2][4];
-                    step_frags<TY>(r, g, byte_pair<(2 * g) & 3>(sc[g >> 1]), byte_pair<(2 * g + 1) & 3>(sc[g >> 1]), lo, hi);
-                    f32x16 S[NJ], H[NJ];
+                    step_frags<TY>(*(const u32x4 *)(wl + (TY == 4 ? 16 : 48) + 32 * g + 16 * hf), qh, g,
+                                   byte_pair<(2 * g) & 3>(sc[g >> 1]), byte_pair<(2 * g + 1) & 3>(sc[g >> 1]), lo, hi);
+                    auto dots = [&](const uint32_t (&f)[2][4], int c, int j) {
+                        const f32x16 S = mfma_f16(f[0], frag(buf, g & 1, c + hf, j), zero16);
+                        return mfma_f16(f[1], frag(buf, g & 1, c + 2 + hf, j), S);
+                    };
+                    if constexpr (TY == 4) {
+                        f32x16 S[NJ], H[NJ];
 #pragma unroll
-                    for (int j = 0; j < NJ; j++) {
-                        S[j] = mfma_f16(lo[0], frag(buf, g, 0 + hf, j), zero16);
-                        S[j] = mfma_f16(lo[1], frag(buf, g, 2 + hf, j), S[j]);
-                    }
+                        for (int j = 0; j < NJ; j++) S[j] = dots(lo, 0, j);
 #pragma unroll
-                    for (int j = 0; j < NJ; j++) {
-                        H[j] = mfma_f16(hi[0], frag(buf, g, 4 + hf, j), zero16);
-                        H[j] = mfma_f16(hi[1], frag(buf, g, 6 + hf, j), H[j]);
-                    }
+                        for (int j = 0; j < NJ; j++) H[j] = dots(hi, 4, j);
 #pragma unroll
-                    for (int j = 0; j < NJ; j++)
+                        for (int j = 0; j < NJ; j++)
 #pragma unroll
-                        for (int v = 0; v < 16; v++) acc[j][v] = __builtin_fmaf(ds[16 * j + v], S[j][v], acc[j][v]);
+                            for (int v = 0; v < 16; v++) acc[j][v] = __builtin_fmaf(ds[16 * j + v], S[j][v], acc[j][v]);
 #pragma unroll
-                    for (int j = 0; j < NJ; j++)
+                        for (int j = 0; j < NJ; j++)
 #pragma unroll
-                        for (int v = 0; v < 16; v++) acc[j][v] = __builtin_fmaf(ds[16 * j + v], H[j][v], acc[j][v]);
-                    if constexpr (TY == 5) {
-                        // mins 2 g, 2 g + 1 against sums 4 g .. 4 g + 3: the other slots are zero
+                            for (int v = 0; v < 16; v++) acc[j][v] = __builtin_fmaf(ds[16 * j + v], H[j][v], acc[j][v]);
+                    } else {
+                        // mins 2 g, 2 g + 1 against sums 4 g .. 4 g + 3: the other slots are zero. One tile at a
+                        // time: both at once do not fit the registers
                         uint32_t bf[4];
 #pragma unroll
                         for (int i = 0; i < 4; i++) bf[i] = (hf == (g >> 1) && (i >> 1) == (g & 1)) ? mf[i] : 0u;
-                        mins(bf);
-                    }
-                };
-                step(std::integral_constant<int, 0>{});
-                step(std::integral_constant<int, 1>{});
-                step(std::integral_constant<int, 2>{});
-                step(std::integral_constant<int, 3>{});
-                if constexpr (TY == 4) mins(mf);
-            } else if constexpr (TY == 3) {
-                // bytes 96..107 (scales), 108..109 (d)
-                uint32_t s[3];
-#pragma unroll
-                for (int i = 0; i < 3; i++) s[i] = __builtin_amdgcn_alignbyte(r.sd[i + 1], r.sd[i], r.sh);
-                const float dw = h2f((uint16_t)(r.sd[3] >> (8 * r.sh)));
-                // chain sign: the products below are negated, so is the scale
-                const f32x32 ds = __builtin_amdgcn_mfma_f32_32x32x1f32(-dw, dxb, zero32, 0, 0, 0);
-                i32x16 I[NJ];
-#pragma unroll
-                for (int j = 0; j < NJ; j++) I[j] = i32x16{};
-#pragma unroll
-                for (int n = 0; n < 2; n++)
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        // raw scale i = 8 n + 2 q + hf (q3k_raw_scales): low nibbles of bytes 0..7 then their
-                        // high nibbles, top bits two by two in bytes 8..11
-                        const int bi = 2 * q + hf;
-                        const int lo = (int)((q < 2 ? s[0] : s[1]) >> (8 * (bi & 3) + (n ? 4 : 0))) & 15;
-                        const int hi2 = (int)(s[2] >> (8 * (bi & 3) + 2 * (2 * n + (q >> 1)))) & 3;
-                        uint32_t f[4];
-                        q3_frag(r, n, q, 32 - (lo | hi2 << 4), f);
-#pragma unroll
-                        for (int j = 0; j < NJ; j++) I[j] = mfma_i8(f, frag(buf, n, 2 * q + hf, j), I[j]);
-                    }
-#pragma unroll
-                for (int j = 0; j < NJ; j++)
-#pragma unroll
-                    for (int v = 0; v < 16; v++) acc[j][v] = __builtin_fmaf((float)I[j][v], ds[16 * j + v], acc[j][v]);
-            } else {
-                // bytes 192..207 (scales), 208..209 (d)
-                uint32_t s[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) s[i] = __builtin_amdgcn_alignbyte(r.sd[i + 1], r.sd[i], r.sh);
-                const float dw = h2f((uint16_t)(r.sd[4] >> (8 * r.sh)));
-                const f32x32 ds = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, dxb, zero32, 0, 0, 0);
-                i32x16 Ih[NJ], Il[NJ];
-#pragma unroll
-                for (int j = 0; j < NJ; j++) Ih[j] = Il[j] = i32x16{};
-#pragma unroll
-                for (int n = 0; n < 2; n++)
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        const int i = 2 * q + hf;   // scale 8 n + i
-                        const int sc = (int)(int8_t)((q < 2 ? s[2 * n] : s[2 * n + 1]) >> (8 * (i & 3)));
-                        uint32_t fh[4], fl[4];
-                        q6_frag(r, n, q, sc, fh, fl);
+                        const f32x32 ms = __builtin_amdgcn_mfma_f32_32x32x1f32(dm, dxb, zero32, 0, 0, 0);
 #pragma unroll
                         for (int j = 0; j < NJ; j++) {
-                            const i32x4 x = frag(buf, n, 2 * q + hf, j);
-                            Ih[j] = mfma_i8(fh, x, Ih[j]);
-                            Il[j] = mfma_i8(fl, x, Il[j]);
+                            const f32x16 S = dots(lo, 0, j), H = dots(hi, 4, j), B = mfma_f16(bf, bsb[j], zero16);
+#pragma unroll
+                            for (int v = 0; v < 16; v++) {
+                                acc[j][v] = __builtin_fmaf(ds[16 * j + v], S[v], acc[j][v]);
+                                acc[j][v] = __builtin_fmaf(ds[16 * j + v], H[v], acc[j][v]);
+                                const float tm = ms[16 * j + v] * B[v];
+                                acc[j][v] = acc[j][v] - tm;
+                            }
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                    }
+                };
+                if (wave_on) {
+                    step(0, std::integral_constant<int, 0>{});
+                    step(0, std::integral_constant<int, 1>{});
+                }
+                stage_sync();
+                if (2 * b + 2 < ns) fetch(0, 2 * b + 2);
+                if (wave_on) {
+                    step(1, std::integral_constant<int, 2>{});
+                    step(1, std::integral_constant<int, 3>{});
+                    if constexpr (TY == 4) mins(mf);
+                }
+            } else if (wave_on) {
+                const int buf = b & 1, sh = 2 * (b & 1);
+                if constexpr (TY == 3) {
+                    Raw3 r;
+                    r.load(wl, hf);
+                    Run sr;   // bytes 96..107 (scales), 108..109 (d)
+                    sr.load(wl + 96);
+                    uint32_t s[3];
+#pragma unroll
+                    for (int i = 0; i < 3; i++) s[i] = sr.get(i, sh);
+                    const float dw = h2f((uint16_t)(sr.w[3] >> (8 * sh)));
+                    // chain sign: the products below are negated, so is the scale
+                    const f32x32 ds = __builtin_amdgcn_mfma_f32_32x32x1f32(-dw, dxb, zero32, 0, 0, 0);
+                    i32x16 I[NJ];
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) I[j] = i32x16{};
+#pragma unroll
+                    for (int n = 0; n < 2; n++)
+#pragma unroll
+                        for (int q = 0; q < 4; q++) {
+                            // raw scale i = 8 n + 2 q + hf (q3k_raw_scales): low nibbles of bytes 0..7 then their
+                            // high nibbles, top bits two by two in bytes 8..11
+                            const int bi = 2 * q + hf;
+                            const int lo = (int)((q < 2 ? s[0] : s[1]) >> (8 * (bi & 3) + (n ? 4 : 0))) & 15;
+                            const int hi2 = (int)(s[2] >> (8 * (bi & 3) + 2 * (2 * n + (q >> 1)))) & 3;
+                            uint32_t f[4];
+                            q3_frag(r, sh, n, q, 32 - (lo | hi2 << 4), f);
+#pragma unroll
+                            for (int j = 0; j < NJ; j++) I[j] = mfma_i8(f, frag(buf, n, 2 * q + hf, j), I[j]);
+                        }
+#pragma unroll
+                    for (int j = 0; j < NJ; j++)
+#pragma unroll
+                        for (int v = 0; v < 16; v++) acc[j][v] = __builtin_fmaf((float)I[j][v], ds[16 * j + v], acc[j][v]);
+                } else {
+                    Run sr;   // bytes 192..207 (scales), 208..209 (d)
+                    sr.load(wl + 192);
+                    uint32_t s[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) s[i] = sr.get(i, sh);
+                    const float dw = h2f((uint16_t)(sr.x >> (8 * sh)));
+                    const f32x32 ds = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, dxb, zero32, 0, 0, 0);
+                    i32x16 Ih[NJ], Il[NJ];
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) Ih[j] = Il[j] = i32x16{};
+#pragma unroll
+                    for (int n = 0; n < 2; n++) {
+                        Raw6 r;
+                        r.load(wl, hf, n);
+#pragma unroll
+                        for (int q = 0; q < 4; q++) {
+                            const int i = 2 * q + hf;   // scale 8 n + i
+                            const int sc = (int)(int8_t)((q < 2 ? s[2 * n] : s[2 * n + 1]) >> (8 * (i & 3)));
+                            uint32_t fh[4], fl[4];
+                            q6_frag(r, sh, q, sc, fh, fl);
+#pragma unroll
+                            for (int j = 0; j < NJ; j++) {
+                                const i32x4 x = frag(buf, n, 2 * q + hf, j);
+                                Ih[j] = mfma_i8(fh, x, Ih[j]);
+                                Il[j] = mfma_i8(fl, x, Il[j]);
+                            }
                         }
                     }
 #pragma unroll
-                for (int j = 0; j < NJ; j++)
+                    for (int j = 0; j < NJ; j++)
 #pragma unroll
-                    for (int v = 0; v < 16; v++) {
-                        const int I = Ih[j][v] * 64 + Il[j][v];
-                        const float tv = (float)I * ds[16 * j + v];
-                        acc[j][v] = acc[j][v] + tv;
-                    }
+                        for (int v = 0; v < 16; v++) {
+                            const int I = Ih[j][v] * 64 + Il[j][v];
+                            const float tv = (float)I * ds[16 * j + v];
+                            acc[j][v] = acc[j][v] + tv;
+                        }
+                }
             }
-        };
-        auto stage_sync = [&]() {
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-        };
-        fetch(0, 0);
-        wload(0);
-        for (int b = 0; b < nb; b++) {
-            stage_sync();   // block b's codes in LDS, every wave done with the other buffer
-            const Raw<TY> cur = raw;
-            const float cdx = dx;
-            i32x4 cbs[NJ];
-#pragma unroll
-            for (int j = 0; j < NJ; j++) cbs[j] = bs[j];
-            if (b + 1 < nb) {
-                fetch((b + 1) & 1, b + 1);
-                wload(b + 1);
-            }
-            compute(b & 1, cur, cdx, cbs);
         }
         if (!wave_on) return;
         // tile j's outputs in this lane: rows 8 q + 4 hf + e (v = 4 q + e), token 32 j + fr
@@ -555,9 +584,12 @@ int kq_gemm_launch(int type, KqGemmArgs a, int64_t ntiles, hipStream_t st) {
     if (a.nseg < 1 || a.nseg > KQG_SEGS || a.nb < 1 || !a.y || !a.x.d || a.ldy % 4 != 0 || (a.res && a.ldr % 4 != 0)) return -1;
     if (((uintptr_t)a.y | (uintptr_t)a.res) % 16 != 0) return -1;
     for (int i = 0; i < a.nseg; i++)
+        if ((uint64_t)a.seg[i].nr * (uint64_t)a.nb * 210 > UINT32_MAX) return -1;   // 32-bit weight offsets
+    for (int i = 0; i < a.nseg; i++)
         if (!a.seg[i].w || a.seg[i].nr < 4 || a.seg[i].nr % 4 != 0 || a.seg[i].off % 4 != 0 || (uintptr_t)a.seg[i].w % 16 != 0) return -1;
     const bool f16 = kqg_f16(type);
     if (f16 ? (!a.x.c16 || !a.x.bs) : !a.x.c8) return -1;
+    if (!f16 && a.nb % 2 != 0) return -1;   // 110- and 210-byte blocks: every row starts on a dword
     if ((uint64_t)a.nt * (uint64_t)a.nb * (f16 ? 512 : 256) > UINT32_MAX) return -1;   // 32-bit code offsets
     const int64_t ny = a.tiles ? ntiles : (a.nt + kqg::BN - 1) / kqg::BN;
     if (ny <= 0) return 0;
