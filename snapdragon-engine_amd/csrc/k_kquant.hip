@@ -880,18 +880,24 @@ __global__ __launch_bounds__(256) void kq_head_norm_kernel(const RunCtl *__restr
     q8K_rows_lds<NL>(s_n, xk);   // the head GEMV's activation
 }
 
+// workgroup (slice of the rows, lane): 16-byte reads of a slice, then one key per workgroup into the lane's (two
+// workgroups of 1024 threads for both lanes' 248320 logits took 77 us, these 5)
+constexpr int AM_WG = 128;
 template <int NL>
-__global__ __launch_bounds__(1024) void kq_argmax_kernel(const RunCtl *__restrict__ ctl, const float *logits, int64_t nv,
-                                                         unsigned long long *amax_key, const uint32_t *ids) {
-    __shared__ unsigned long long red[16];
+__global__ __launch_bounds__(256) void kq_argmax_kernel(const RunCtl *__restrict__ ctl, const float *logits, int64_t nv,
+                                                        unsigned long long *amax_key, const uint32_t *ids) {
+    __shared__ unsigned long long red[4];
     if (!ctl->active) return;
-    const int l = blockIdx.x, t = threadIdx.x;
+    const int l = blockIdx.y, t = threadIdx.x;
     if (l >= ctl->nl || !((ctl->head_mask >> l) & 1)) return;
     float best = -__builtin_inff();
     int64_t bi = -1;
-    for (int64_t r = t; r < nv; r += 1024) {
-        const float v = logits[(int64_t)l * nv + r];
-        if (v > best) { best = v; bi = r; }
+    for (int64_t r = 4 * (blockIdx.x * 256 + t); r < nv; r += 4 * 256 * AM_WG) {
+        const float4 v = *(const float4 *)(logits + (int64_t)l * nv + r);
+        if (v.x > best) { best = v.x; bi = r; }
+        if (v.y > best) { best = v.y; bi = r + 1; }
+        if (v.z > best) { best = v.z; bi = r + 2; }
+        if (v.w > best) { best = v.w; bi = r + 3; }
     }
     // a restricted draft head's rows are ascending token ids: the first maximum by row is the first by id
     const uint32_t id = bi < 0 ? 0u : (ids ? ids[bi] : (uint32_t)bi);
@@ -904,7 +910,7 @@ __global__ __launch_bounds__(1024) void kq_argmax_kernel(const RunCtl *__restric
     __syncthreads();
     if (t == 0) {
         unsigned long long k = 0ull;
-        for (int i = 0; i < 16; i++) k = red[i] > k ? red[i] : k;
+        for (int i = 0; i < 4; i++) k = red[i] > k ? red[i] : k;
         if (k) atomicMax(&amax_key[l], k);
     }
 }
@@ -1032,7 +1038,7 @@ int launch_kq_head(const RunCtl *ctl, const ModelRt &m, const float *norm_w, con
         default: rc = kq::vl_gemv_type<6>(o.w, nb, o.rows, b.xk, OXE_NL, b.logits, st); break;
     }
     if (rc != 1) return -2;
-    hipLaunchKernelGGL(kq::kq_argmax_kernel<OXE_NL>, dim3(OXE_NL), dim3(1024), 0, st, ctl, b.logits, o.rows, b.amax_key, ids);
+    hipLaunchKernelGGL(kq::kq_argmax_kernel<OXE_NL>, dim3(kq::AM_WG, OXE_NL), dim3(256), 0, st, ctl, b.logits, o.rows, b.amax_key, ids);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
