@@ -93,8 +93,9 @@ __global__ __launch_bounds__(gm::NT, 3) void gemm_q8_kernel(GemmArgs a, int vec4
     if (a.tiles) {
         if (a.tile_count && (int)blockIdx.y >= *a.tile_count) return;   // uniform: before any barrier
         const int4 tl = a.tiles[blockIdx.y];
-        wq += (int64_t)tl.x * a.wq_stride;
-        wd += (int64_t)tl.x * a.wd_stride;
+        const bool last = a.last > 0 && tl.x == a.last;
+        wq = last ? a.wq_last : wq + (int64_t)tl.x * a.wq_stride;
+        wd = last ? a.wd_last : wd + (int64_t)tl.x * a.wd_stride;
         p0 = tl.y;
         pn = tl.z;
     } else {
@@ -497,7 +498,7 @@ extern "C" {
 int oxe_hip_gemm_q8_0(int64_t k, int64_t nr, int64_t nt, const int8_t *wq, const uint16_t *wd, const int8_t *xq,
                       const uint16_t *xd, float *y, int64_t ldy, void *stream) {
     if (nt <= 0) return -1;
-    oxe::GemmArgs a{wq, wd, xq, xd, y, nullptr, nr, nt, k, ldy, 0, nullptr, 0, 0, nullptr};
+    oxe::GemmArgs a{wq, wd, xq, xd, y, nullptr, nr, nt, k, ldy, 0, nullptr, 0, 0, nullptr, nullptr, nullptr, nullptr, 0};
     return oxe::gemm_launch(a, 0, (hipStream_t)stream);
 }
 

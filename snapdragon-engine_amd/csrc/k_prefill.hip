@@ -77,9 +77,8 @@ __global__ __launch_bounds__(256) void conv_kernel(const float *proj, int T, con
     }
     cy[t * NCH + c] = v_silu(conv4_pf(s[0], s[1], s[2], s[3], cw));
 }
-// the window after the chunk: the last three inputs (for T < 3 partly the older state)
-__global__ __launch_bounds__(256) void conv_state_kernel(const float *proj, int T, float *state) {
-    const int c = blockIdx.x * 256 + threadIdx.x;
+// the window of channel c after the chunk: the last three inputs (for T < 3 partly the older state)
+OXE_DEV void conv_state(const float *proj, int T, float *state, int c) {
     float *st = state + (int64_t)c * (KC - 1);
     float n[KC - 1];
 #pragma unroll
@@ -92,10 +91,17 @@ __global__ __launch_bounds__(256) void conv_state_kernel(const float *proj, int 
 }
 
 // l2 norms of q and k (oxe_gdn_l2_norm_f32: rms_norm with eps/n, then * 1/sqrt(n)), one wave per
-// (token, key head, q|k), in place; the gates of (token, value head) (engine.rs:2509-2524)
+// (token, key head, q|k), in place; the gates of (token, value head) (engine.rs:2509-2524). Columns of workgroups
+// past the tokens move the conv window on (conv_kernel has read the old one; a launch of its own took 4.7 us)
+constexpr int PREP_Y = 8, PREP_CONV = NCH / 256 / PREP_Y;
 __global__ __launch_bounds__(256) void dn_prep_kernel(float *cy, const float *proj, const float *dt_bias,
-                                                      const float *ssm_a, float eps, float *gg, float *gb) {
+                                                      const float *ssm_a, float eps, float *gg, float *gb, int T,
+                                                      float *conv_st) {
     const int64_t t = blockIdx.x;
+    if (t >= T) {   // uniform
+        conv_state(proj, T, conv_st, (((int)t - T) * PREP_Y + blockIdx.y) * 256 + threadIdx.x);
+        return;
+    }
     const int w = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;   // 0..31
     const int kh = w >> 1;
     float *xv = cy + t * NCH + ((w & 1) ? NKH * DS : 0) + kh * DS;
@@ -765,57 +771,52 @@ __global__ __launch_bounds__(256) void route_kernel(const float *lg, int T, int3
     if (lane == 0 && ro[w].tie) atomicAdd(tie_count, 1u);
 }
 
-// (token, rank) pairs grouped by expert: counts, then (one workgroup) offsets and the 64-pair tiles
-// of every expert, then the scatter. The order of pairs inside an expert's group is free: every
-// (pair, row) result of the grouped GEMMs is independent of its neighbours.
-constexpr int MO_CNT = 0, MO_OFF = NEXP, MO_FILL = 2 * NEXP, MO_NT = 3 * NEXP, MO_WORDS = 3 * NEXP + 1;
-__global__ void moe_count_kernel(const int32_t *ids, int np, int32_t *mo) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < np) atomicAdd(&mo[MO_CNT + ids[i]], 1);
-}
-__global__ __launch_bounds__(NEXP) void moe_tiles_kernel(int32_t *mo, int4 *tiles) {
-    __shared__ int s_c[NEXP], s_t[NEXP];
-    const int e = threadIdx.x;
-    const int c = mo[MO_CNT + e], nt = (c + 63) / 64;
-    s_c[e] = c;
-    s_t[e] = nt;
+// (token, rank) pairs grouped by expert, by one workgroup with the counters in LDS: counts, offsets and the 64-pair
+// tiles of every expert, then the scatter. The order of pairs inside an expert's group is free: every (pair, row)
+// result of the grouped GEMMs is independent of its neighbours. (A memset, a count, a tile and a scatter kernel took
+// 18 us at 61 tokens and 27 us at 2048, this 5 and 17.)
+// sh_rows > 0: the shared expert joins the groups as expert NEXP, its rows np + t for tokens t < sh_rows.
+constexpr int MO_NT = 0, MO_WORDS = 1;   // words of mo: the tiles
+constexpr int MO_T = 1024;
+__global__ __launch_bounds__(MO_T) void moe_group_kernel(const int32_t *ids, int np, int sh_rows, int32_t *mo, int4 *tiles,
+                                                         int32_t *ptok, int32_t *pair_of) {
+    __shared__ int s_n[NEXP], s_c[NEXP], s_t[NEXP], s_o[NEXP];
+    const int t = threadIdx.x;
+    if (t < NEXP) s_n[t] = 0;
+    __syncthreads();
+    for (int i = t; i < np; i += MO_T) atomicAdd(&s_n[ids[i]], 1);
+    __syncthreads();
+    const int c = t < NEXP ? s_n[t] : 0, nt = (c + 63) / 64;
+    if (t < NEXP) {
+        s_c[t] = c;
+        s_t[t] = nt;
+    }
     __syncthreads();
     for (int d = 1; d < NEXP; d <<= 1) {
-        const int a = e >= d ? s_c[e - d] : 0, b = e >= d ? s_t[e - d] : 0;
+        const int a = t < NEXP && t >= d ? s_c[t - d] : 0, b = t < NEXP && t >= d ? s_t[t - d] : 0;
         __syncthreads();
-        s_c[e] += a;
-        s_t[e] += b;
+        if (t < NEXP) {
+            s_c[t] += a;
+            s_t[t] += b;
+        }
         __syncthreads();
     }
-    const int off = s_c[e] - c, tb = s_t[e] - nt;
-    mo[MO_OFF + e] = off;
-    mo[MO_FILL + e] = 0;
-    for (int s = 0; s < nt; s++) tiles[tb + s] = make_int4(e, off + 64 * s, min(64, c - 64 * s), 0);
-    if (e == NEXP - 1) mo[MO_NT] = s_t[e];
-}
-__global__ void moe_scatter_kernel(const int32_t *ids, int np, int32_t *mo, int32_t *ptok, int32_t *pair_of) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= np) return;
-    const int e = ids[i];
-    const int p = mo[MO_OFF + e] + atomicAdd(&mo[MO_FILL + e], 1);
-    ptok[p] = i / KUSED;
-    pair_of[i] = p;
-}
-
-// swiglu (ggml_vec_swiglu_f32: silu(gate) * up) of a gate/up output row with the 16-row interleave
-// (8 gate rows, then 8 up rows) and the Q8_0 of the 512 values: one workgroup per row
-__global__ __launch_bounds__(256) void swiglu_quant_kernel(const float *gu, int8_t *hq, uint16_t *hd) {
-    const int64_t r = blockIdx.x;
-    const float *g = gu + r * (2 * FF);
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const int i = threadIdx.x + 256 * k, tl = i >> 3, rr = i & 7;
-        const float h = v_silu(g[tl * 16 + rr]) * g[tl * 16 + 8 + rr];
-        float dd;
-        const uint32_t word = quant32_lanes(h, &dd);
-        if ((i & 3) == 0) *(uint32_t *)(hq + r * FF + i) = word;
-        if ((i & 31) == 0) hd[r * (FF / 32) + i / 32] = f2h(dd);
+    const int ntile = s_t[NEXP - 1];
+    if (t < NEXP) {
+        const int off = s_c[t] - c, tb = s_t[t] - nt;
+        s_o[t] = off;
+        for (int s = 0; s < nt; s++) tiles[tb + s] = make_int4(t, off + 64 * s, min(64, c - 64 * s), 0);
     }
+    const int nsh = (sh_rows + 63) / 64;
+    for (int s = t; s < nsh; s += MO_T) tiles[ntile + s] = make_int4(NEXP, np + 64 * s, min(64, sh_rows - 64 * s), 0);
+    if (t == 0) mo[MO_NT] = ntile + nsh;
+    __syncthreads();
+    for (int i = t; i < np; i += MO_T) {
+        const int p = atomicAdd(&s_o[ids[i]], 1);
+        ptok[p] = i / KUSED;
+        pair_of[i] = p;
+    }
+    for (int i = t; i < sh_rows; i += MO_T) ptok[np + i] = i;
 }
 
 // combine (engine.rs:3591-3601): m = d_0 w_0, m = m + d_j w_j (j = 1..7), f = m + d_sh g_sh,
@@ -898,14 +899,15 @@ int Engine::pf_alloc(int T) {
         pfb.ids = alloc<int32_t>(np);
         pfb.wts = alloc<float>(np);
         pfb.mo = alloc<int32_t>(pf::MO_WORDS);
-        pfb.ptok = alloc<int32_t>(np);
+        pfb.ptok = alloc<int32_t>(np + T);
         pfb.pair_of = alloc<int32_t>(np);
-        pfb.max_tiles = (int)(np / 64 + NEXP);
+        pfb.max_tiles = (int)(np / 64 + NEXP + (T + 63) / 64);
         pfb.tiles = alloc<int4>((size_t)pfb.max_tiles);
-        pfb.gu = alloc<float>(np * 2 * FF);
-        pfb.hq = alloc<int8_t>(np * FF);
-        pfb.hd = alloc<uint16_t>(np * (FF / 32));
-        pfb.dout = alloc<float>(np * E);
+        const size_t nr = np + T;   // rows of the routed pairs and of the shared expert
+        pfb.gu = alloc<float>(nr * 2 * FF);
+        pfb.hq = alloc<int8_t>(nr * FF);
+        pfb.hd = alloc<uint16_t>(nr * (FF / 32));
+        pfb.dout = alloc<float>(nr * E);
         pfb.sh = alloc<float>((size_t)T * E);
         pfb.tok = alloc<uint32_t>((size_t)T);
         if (kq) {
@@ -971,10 +973,13 @@ int Engine::pf_chunk(const uint32_t *toks, int T, float *h_out) {
         return r;
     };
     auto grouped = [&](const Q8W &w, int64_t rows, int64_t k, const int8_t *xq, const uint16_t *xd, const int32_t *xrow,
-                       float *y) {
+                       float *y, const Q8W *sh) {
         GemmArgs g{};
         g.wq = w.q; g.wd = w.d; g.xq = xq; g.xd = xd; g.y = y;
-        g.nr = rows; g.nt = np; g.k = k; g.ldy = rows;
+        g.nr = rows; g.nt = np + (sh ? T : 0); g.k = k; g.ldy = rows;
+        if (sh) {
+            g.wq_last = sh->q; g.wd_last = sh->d; g.last = NEXP;
+        }
         g.tiles = pfb.tiles; g.wq_stride = rows * k; g.wd_stride = rows * (k / 32); g.xrow = xrow;
         g.tile_count = pfb.mo + MO_NT;
         probe(K_PF_GEMM); probe(K_PF_EXPERT);
@@ -1042,9 +1047,8 @@ int Engine::pf_chunk(const uint32_t *toks, int T, float *h_out) {
             float *cs = m.conv_state + (int64_t)cur * conv_slot + (int64_t)w.index * NCH * (KC - 1);
             float *ss = m.ssm_state + (int64_t)cur * ssm_slot + (int64_t)w.index * NVH * HV * HV;
             hipLaunchKernelGGL(conv_kernel, dim3(NCH / 256, T), dim3(256), 0, st, pfb.proj, T, w.conv, cs, pfb.cy);
-            hipLaunchKernelGGL(conv_state_kernel, dim3(NCH / 256), dim3(256), 0, st, pfb.proj, T, cs);
-            hipLaunchKernelGGL(dn_prep_kernel, dim3(T, 8), dim3(256), 0, st, pfb.cy, pfb.proj, w.dt_bias, w.ssm_a, eps,
-                               pfb.gg, pfb.gb);
+            hipLaunchKernelGGL(dn_prep_kernel, dim3(T + PREP_CONV, PREP_Y), dim3(256), 0, st, pfb.cy, pfb.proj, w.dt_bias, w.ssm_a,
+                               eps, pfb.gg, pfb.gb, T, cs);
             probe(K_PF_DELTA);
             hipLaunchKernelGGL(delta_kernel, dim3(NVH * 8), dim3(256), 0, st, pfb.cy, pfb.gg, pfb.gb, ss, pfb.o, T);
             probe(K_PF_DELTA);
@@ -1102,11 +1106,19 @@ int Engine::pf_chunk(const uint32_t *toks, int T, float *h_out) {
                 h = forms(pfb.kh, dn, 1);
                 return kq_pf_swiglu_q8_K(pfb.gu, split, rows, h, st);
             }
-            if (split) return kq_pf_swiglu_q8_0(pfb.gu, true, rows, pfb.hq, pfb.hd, st);
-            hipLaunchKernelGGL(swiglu_quant_kernel, dim3((unsigned)rows), dim3(256), 0, st, pfb.gu, pfb.hq, pfb.hd);
-            return 0;
+            return kq_pf_swiglu_q8_0(pfb.gu, split, rows, pfb.hq, pfb.hd, st);
         };
         KqAct h{};
+        // routed experts: pairs grouped by expert, 64-pair tiles built on the device. With Q8_0 matrices throughout the
+        // shared expert is one more group: its rows fill the experts' launches and need none of their own
+        const bool join = !kegu && !ksgu && !kedn && !ksdn;
+        hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(MO_T), 0, st, pfb.ids, np, join ? T : 0, pfb.mo, pfb.tiles, pfb.ptok,
+                           pfb.pair_of);
+        if (join) {
+            if ((rc = grouped(w.exp_gu, 2 * FF, E, pfb.xq, pfb.xd, pfb.ptok, pfb.gu, &w.shexp_gu))) return rc;
+            if ((rc = kq_pf_swiglu_q8_0(pfb.gu, false, np + T, pfb.hq, pfb.hd, st))) return rc;
+            if ((rc = grouped(w.exp_down, E, FF, pfb.hq, pfb.hd, nullptr, pfb.dout, &w.shexp_down))) return rc;
+        } else {
         // shared expert over all tokens
         if (ksgu) rc = kgemm(sgu, 2, E, xa, pfb.gu, 2 * FFSH, nullptr, T, nullptr, false);
         else rc = gemm(w.shexp_gu, pfb.xq, pfb.xd, E, pfb.gu, 2 * FFSH, nullptr, T);
@@ -1115,21 +1127,16 @@ int Engine::pf_chunk(const uint32_t *toks, int T, float *h_out) {
         if (ksdn) rc = kgemm(sdn, 1, FFSH, h, pfb.sh, E, nullptr, T, nullptr, false);
         else rc = gemm(w.shexp_down, pfb.hq, pfb.hd, FFSH, pfb.sh, E, nullptr, T);
         if (rc) return rc;
-        // routed experts: pairs grouped by expert, 64-pair tiles built on the device
-        if (hipMemsetAsync(pfb.mo, 0, NEXP * 4, st) != hipSuccess) return -2;
-        hipLaunchKernelGGL(moe_count_kernel, dim3((np + 255) / 256), dim3(256), 0, st, pfb.ids, np, pfb.mo);
-        hipLaunchKernelGGL(moe_tiles_kernel, dim3(1), dim3(NEXP), 0, st, pfb.mo, pfb.tiles);
-        hipLaunchKernelGGL(moe_scatter_kernel, dim3((np + 255) / 256), dim3(256), 0, st, pfb.ids, np, pfb.mo, pfb.ptok,
-                           pfb.pair_of);
         if (kegu) rc = kgemm(egu, 2, E, xa, pfb.gu, 2 * FF, nullptr, T, pfb.ptok, true);
-        else rc = grouped(w.exp_gu, 2 * FF, E, pfb.xq, pfb.xd, pfb.ptok, pfb.gu);
+        else rc = grouped(w.exp_gu, 2 * FF, E, pfb.xq, pfb.xd, pfb.ptok, pfb.gu, nullptr);
         if (rc) return rc;
         if ((rc = swiglu(kegu, edn, np, h))) return rc;
         if (kedn) rc = kgemm(edn, 1, FF, h, pfb.dout, E, nullptr, np, nullptr, true);
-        else rc = grouped(w.exp_down, E, FF, pfb.hq, pfb.hd, nullptr, pfb.dout);
+        else rc = grouped(w.exp_down, E, FF, pfb.hq, pfb.hd, nullptr, pfb.dout, nullptr);
         if (rc) return rc;
+        }
         hipLaunchKernelGGL(combine_kernel, dim3((unsigned)(((int64_t)T * E + 255) / 256)), dim3(256), 0, st, pfb.dout,
-                           pfb.pair_of, pfb.wts, pfb.sh, pfb.sg, pfb.x1, pfb.x, T);
+                           pfb.pair_of, pfb.wts, join ? pfb.dout + (int64_t)np * E : pfb.sh, pfb.sg, pfb.x1, pfb.x, T);
         if (hipGetLastError() != hipSuccess) return -2;
     }
     // h_nextn of every token (output norm of x2), the LM head of the last token

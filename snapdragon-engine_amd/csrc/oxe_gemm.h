@@ -21,6 +21,9 @@ struct GemmArgs {
     int64_t wq_stride, wd_stride;
     const int32_t *xrow;
     const int32_t *tile_count;
+    const int8_t *wq_last;     // grouped: weights of group `last` (0: none) outside the run of the others
+    const uint16_t *wd_last;
+    int32_t last;
 };
 
 // rows of y: plain -> nt token rows; grouped -> the tiles' rows (ntiles tiles). 0, -1 (bad shape), -2.
