@@ -19,24 +19,18 @@ constexpr int Q8K_QS = 4, Q8K_BS = 260;
 // (v: this lane's four values; every lane of one wave) the lane's codes; returns d
 OXE_DEV float q8K_codes(const float (&v)[4], int lane, int (&q)[4]) {
     float am = 0.0f, mx = 0.0f;
-    int idx = QK;
     for (int e = 0; e < 4; e++) {
         const float ax = fabsf(v[e]);
         if (ax > am) {
             am = ax;
             mx = v[e];
-            idx = 4 * lane + e;
         }
     }
-    for (int m = 32; m >= 1; m >>= 1) {
-        const float oa = shfl_xor_f(am, m), om = shfl_xor_f(mx, m);
-        const int oi = shfl_xor_i(idx, m);
-        if (oa > am || (oa == am && oi < idx)) {
-            am = oa;
-            mx = om;
-            idx = oi;
-        }
-    }
+    // the wave's largest magnitude by lane moves, then the first lane that holds it (lanes hold values in order)
+    const float top = wave_max_any(am);
+    const unsigned long long at = __ballot(am == top);
+    mx = readlane_f(mx, __builtin_ctzll(at));
+    am = top;
     q[0] = q[1] = q[2] = q[3] = 0;
     if (am == 0.0f) return 0.0f;
     const float iscale = -127.f / mx;
@@ -54,8 +48,8 @@ OXE_DEV uint32_t pack4(const int (&q)[4]) {
 // the lane's sum of 16 codes (every lane of four holds it)
 OXE_DEV int sum16(const int (&q)[4]) {
     int s = q[0] + q[1] + q[2] + q[3];
-    s += shfl_xor_i(s, 1);
-    s += shfl_xor_i(s, 2);
+    s += dpp_i<DPP_XOR1>(s);
+    s += dpp_i<DPP_XOR2>(s);
     return s;
 }
 // the same into a ggml block_q8_K (xb: the block's 256 values)
