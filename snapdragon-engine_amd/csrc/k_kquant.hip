@@ -575,6 +575,27 @@ OXE_DEV void stage_q8k(const uint8_t *y, int nblk, uint32_t *yh, float *yd) {
     for (int i = threadIdx.x; i < nblk; i += blockDim.x) yd[i] = *(const float *)(y + (int64_t)i * Q8K_BYTES);
 }
 
+// the same with a workgroup of T threads and NBLK blocks, every load in flight at once
+template <int T, int NBLK>
+OXE_DEV void stage_q8k_all(const uint8_t *y, uint32_t *yh, float *yd) {
+    constexpr int N = NBLK * 2 * 36, I = (N + T - 1) / T;
+    static_assert(NBLK <= T, "one scale per thread");
+    uint32_t v[I];
+#pragma unroll
+    for (int k = 0; k < I; k++) {
+        const int i = min((int)threadIdx.x + T * k, N - 1), wd = i % 36, hb = i / 36, h = hb & 1;
+        const uint32_t *src = (const uint32_t *)(y + (int64_t)(hb >> 1) * Q8K_BYTES);
+        v[k] = wd < 32 ? src[1 + 32 * h + wd] : src[65 + 4 * h + (wd - 32)];
+    }
+    const float d = *(const float *)(y + (int64_t)min((int)threadIdx.x, NBLK - 1) * Q8K_BYTES);
+#pragma unroll
+    for (int k = 0; k < I; k++) {
+        const int i = min((int)threadIdx.x + T * k, N - 1);
+        yh[i / 36 * YH + i % 36] = v[k];
+    }
+    if (threadIdx.x < NBLK) yd[threadIdx.x] = d;
+}
+
 OXE_DEV uint32_t ordered_bits(float f) {
     const uint32_t u = __builtin_bit_cast(uint32_t, f);
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
@@ -633,6 +654,9 @@ __global__ __launch_bounds__(256) void ba_f32_kernel(const RunCtl *__restrict__ 
 // t / 16 % 8, half block t % 16) forms its half block's integers for every lane; threads t % 16 < NL
 // then run lane t % 16's chain over the row's 8 blocks, gate and up at once; then silu(g) * u
 // (ggml_v_silu, as swiglu) for every lane that routed to the expert (the shared expert: every lane).
+// A tile's rows are one run of bytes per matrix: they come as whole lines, before the activations, and are read from
+// LDS (each thread reading its half block from global memory after the activations, 64 threads 72 bytes apart: 18.4 us a
+// launch with Q4_K experts of two lanes, 14.2 so). Bound by the latency of one round of workgroups.
 struct KqGuArgs {
     const uint8_t *xk;          // [NL][E / 256] q8_K blocks of xn
     RawW gate, up, sh_gate, sh_up;
@@ -644,40 +668,51 @@ struct KqGuArgs {
 };
 constexpr int GU_NB = shp::E / QK;   // 8 blocks per row
 constexpr int GU_R = 8;              // rows per workgroup
+constexpr int GU_LD = (GU_R * GU_NB * 210 / 16 + 127) / 128;   // 16-byte loads per thread: a tile of one matrix, Q6_K's blocks
 static_assert(GU_NB * 2 == 16 && shp::FF == shp::FFSH, "16 half blocks per row; one tiling for both");
 
 template <int NL>
 __global__ __launch_bounds__(256) void kq_gu_kernel(const RunCtl *__restrict__ ctl, KqGuArgs a) {
     constexpr int RS = (NL * RES_MAX) | 1;
+    extern __shared__ __align__(16) uint8_t gu_w[];   // the gate rows, then the up rows
     __shared__ uint32_t yh[NL * GU_NB * 2 * YH];
     __shared__ float yd[NL * GU_NB];
     __shared__ int res[256 * RS];
     __shared__ float s_gu[2][GU_R][NL];
-    if (!ctl->active) return;
-    const int nl = ctl->nl, t = threadIdx.x, which = t >> 7, ri = (t >> 4) & (GU_R - 1), hu = t & 15;
+    const int t = threadIdx.x, which = t >> 7, ri = (t >> 4) & (GU_R - 1), hu = t & 15;
     const int u = blockIdx.x / (shp::FF / GU_R), tile = blockIdx.x % (shp::FF / GU_R);
     const bool sh = u == OXE_MAX_UNION;
+    // one round trip for all that says which rows to read
+    const int active = ctl->active, nl = ctl->nl, nu = a.uni[0];
+    int e = a.uni[1 + (sh ? 0 : u)];
+    if (!active) return;
     if (a.do_exp && blockIdx.x == 0 && t == 0) {
-        atomicAdd(a.stats, (uint32_t)a.uni[0]);
+        atomicAdd(a.stats, (uint32_t)nu);
         atomicAdd(a.stats + 1, 1u);
     }
     if (sh ? !a.do_sh : !a.do_exp) return;
-    int e = 0;
-    if (!sh) {
-        int nu = a.uni[0];
-        nu = nu < 0 ? 0 : (nu > OXE_MAX_UNION ? OXE_MAX_UNION : nu);
-        if (u >= nu) return;
-        e = a.uni[1 + u];
-        e = e < 0 ? 0 : (e >= shp::NEXP ? shp::NEXP - 1 : e);
-    }
-    stage_q8k(a.xk, NL * GU_NB, yh, yd);
+    if (!sh && u >= nu) return;
+    e = sh || e < 0 ? 0 : (e >= shp::NEXP ? shp::NEXP - 1 : e);
+    const RawW &W = sh ? (which ? a.sh_up : a.sh_gate) : (which ? a.up : a.gate);
+    const int type = W.type, rs = res_of(type), rb = (int)raw_row_bytes(W), n16 = GU_R * rb / 16;
+    const u32x4 *src = (const u32x4 *)(W.w + ((int64_t)e * W.rows + tile * GU_R) * rb);
+    u32x4 pf[GU_LD];
+#pragma unroll
+    for (int k = 0; k < GU_LD; k++) pf[k] = __builtin_nontemporal_load(src + min((t & 127) + 128 * k, n16 - 1));
+    __builtin_amdgcn_sched_barrier(0);   // the weights before the activations
+    stage_q8k_all<256, NL * GU_NB>(a.xk, yh, yd);
+    int slot = -1;
+    if (which == 0 && hu < NL && hu < nl && !sh)
+#pragma unroll
+        for (int jj = 0; jj < shp::KUSED; jj++)
+            if (a.route_ids[hu * shp::KUSED + jj] == e) slot = jj;
+    uint8_t *wl = gu_w + (which ? GU_R * (int)raw_row_bytes(sh ? a.sh_gate : a.gate) : 0);
+#pragma unroll
+    for (int k = 0; k < GU_LD; k++) ((u32x4 *)wl)[min((t & 127) + 128 * k, n16 - 1)] = pf[k];   // clamped: same bytes
     __syncthreads();
     const int row = tile * GU_R + ri;
     {
-        const RawW &W = sh ? (which ? a.sh_up : a.sh_gate) : (which ? a.up : a.gate);
-        const int type = W.type, rs = res_of(type);
-        const int64_t rb = raw_row_bytes(W);
-        const uint8_t *wr = W.w + ((int64_t)e * W.rows + row) * rb;
+        const uint8_t *wr = wl + ri * rb;
         unit_rt<NL>(type, wr + (hu >> 1) * kq_block_bytes(type), YView{yh + (2 * (hu >> 1) + (hu & 1)) * YH, GU_NB * 2 * YH},
                     hu & 1, res + t * RS);
         __syncthreads();
@@ -693,24 +728,20 @@ __global__ __launch_bounds__(256) void kq_gu_kernel(const RunCtl *__restrict__ c
     }
     if (which == 0 && hu < NL && hu < nl) {
         const float h = v_silu(s_gu[0][ri][hu]) * s_gu[1][ri][hu];
-        if (sh) {
-            a.hsh[(int64_t)hu * shp::FFSH + row] = h;
-        } else {
-            int j = -1;
-            for (int jj = 0; jj < shp::KUSED; jj++)
-                if (a.route_ids[hu * shp::KUSED + jj] == e) j = jj;
-            if (j >= 0) a.hexp[((int64_t)hu * shp::KUSED + j) * shp::FF + row] = h;
-        }
+        if (sh) a.hsh[(int64_t)hu * shp::FFSH + row] = h;
+        else if (slot >= 0) a.hexp[((int64_t)hu * shp::KUSED + slot) * shp::FF + row] = h;
     }
 }
 
-// ---- MoE down + combine with any mix of K-quant and Q8_0 down matrices: workgroup = 16 output
+// ---- MoE down + combine with any mix of K-quant and Q8_0 down matrices: workgroup = 8 output
 // rows; units 0..nu-1 the union's experts, unit OXE_MAX_UNION the shared expert. Each (unit, lane,
 // row) value is that matrix's row dot with the lane's h (slot j of the lane's top-k, or the shared
-// h): K-quants on h's q8_K blocks (2 per row of 512), four units per pass with 64 threads each
-// (row, half block); Q8_0 on h quantised to Q8_0 in LDS, one thread per (unit, lane, row) running
-// the block chain. Then the reference's combine (engine.rs:3591-3601):
-// m = d0 w0; m += dj wj; f = m + dsh * g; x2 = f + x1.
+// h): K-quants on h's q8_K blocks (2 per row of 512), Q8_0 on h quantised to Q8_0 in LDS. Then the
+// reference's combine (engine.rs:3591-3601): m = d0 w0; m += dj wj; f = m + dsh * g; x2 = f + x1.
+// 32 threads per unit, every unit at once: a unit's 8 rows are one run of bytes, requested as whole lines before
+// anything else and read from LDS, so the launch waits for memory once (256 workgroups, one per CU, whose 125 KB
+// of LDS and registers nothing else wants). Eight units a pass from global memory, the Q8_0 unit's blocks by one
+// thread per row: 17.2 us a launch with Q5_K experts and a Q8_0 shared matrix, two lanes; 8.8 so.
 struct KqDownArgs {
     const int32_t *uni, *route_ids;
     const float *route_w, *sh_gate;
@@ -726,53 +757,75 @@ constexpr int DN_R = 8;                      // output rows per workgroup (E / 8
 constexpr int DN_NB = shp::FF / QK;          // 2 blocks per down row
 constexpr int DN_U = OXE_MAX_UNION + 1;
 constexpr int DN_A = shp::KUSED + 1;         // activation rows per lane: the k slots, then the shared h
+constexpr int DN_T = 64 * ((DN_U + 1) / 2);  // 32 threads per unit
+constexpr int DN_SLAB = DN_R * (shp::FF + shp::FF / 16);   // most bytes of a unit's rows: Q8_0 codes, then scales
+constexpr int DN_LD = (DN_SLAB / 16 + 31) / 32;            // 16-byte loads per thread of a unit
 
 template <int NL>
-__global__ __launch_bounds__(256) void kq_down_kernel(const RunCtl *__restrict__ ctl, KqDownArgs a) {
+__global__ __launch_bounds__(DN_T) void kq_down_kernel(const RunCtl *__restrict__ ctl, KqDownArgs a) {
     constexpr int RS = (NL * RES_MAX) | 1;   // odd per-thread stride of the unit integers
+    constexpr int QB = shp::FF / 32;         // Q8_0 blocks of a row
+    static_assert(DN_R == 8 && OXE_MAX_UNION % 2 == 0, "32 threads per unit; the shared unit in a wave of its own");
+    static_assert(DN_SLAB % 16 == 0 && DN_SLAB >= DN_R * DN_NB * 210 && 32 * RS >= NL * DN_R * QB, "a unit's LDS");
+    __shared__ __align__(16) uint8_t s_wl[DN_U][DN_SLAB];
     __shared__ uint32_t yh[NL * DN_A * DN_NB * 2 * YH];
     __shared__ float yd[NL * DN_A * DN_NB];
-    __shared__ int8_t s_q[NL * DN_A][shp::FF];
-    __shared__ uint16_t s_d[NL * DN_A][shp::FF / 32];
-    __shared__ int res[256 * RS];
+    __shared__ __align__(16) int8_t s_q[NL * DN_A][shp::FF];
+    __shared__ uint16_t s_d[NL * DN_A][QB];
+    __shared__ int res[DN_T * RS];
     __shared__ float s_dn[NL][DN_A][DN_R];
-    __shared__ int32_t s_e[DN_U], s_slot[DN_U][NL];
+    __shared__ int32_t s_slot[DN_U][NL];
     __shared__ float s_w[NL][shp::KUSED], s_sg[NL];
-    if (!ctl->active) return;
-    const int nl = ctl->nl, t = threadIdx.x;
+    const int t = threadIdx.x, u = t >> 5, ti = t & 31;
+    const bool shu = __builtin_amdgcn_readfirstlane(t >> 6) == OXE_MAX_UNION / 2;
+    const int active = ctl->active, nl = ctl->nl, nu = a.uni[0], e0 = shu ? 0 : a.uni[1 + u];
+    if (!active) return;
     const int64_t row0 = (int64_t)blockIdx.x * DN_R;
+    const bool live = u < DN_U && (shu || u < nu);
+    const RawW &W = shu ? a.sh_down_r : a.exp_down_r;
+    const int type = W.type, bb = type != 8 ? kq_block_bytes(type) : 0;
+    const int64_t e = e0 < 0 ? 0 : (e0 < shp::NEXP ? e0 : shp::NEXP - 1);   // slots below compare the unclamped id
+    // the unit's 8 rows (one run of bytes), on their way before anything else
+    u32x4 pf[DN_LD];
+    if (live) {
+        if (type == 8) {
+            const Q8W &Q = shu ? a.shexp_down : a.exp_down;
+            const u32x4 *q = (const u32x4 *)(Q.q + (e * shp::E + row0) * shp::FF), *d = (const u32x4 *)(Q.d + (e * shp::E + row0) * QB);
+#pragma unroll
+            for (int k = 0; k < DN_LD - 1; k++) pf[k] = __builtin_nontemporal_load(q + ti + 32 * k);
+            pf[DN_LD - 1] = __builtin_nontemporal_load(d + (ti & 15));
+        } else {
+            const u32x4 *src = (const u32x4 *)(W.w + (e * W.rows + row0) * raw_row_bytes(W));   // 16 blocks: bb chunks
+#pragma unroll
+            for (int k = 0; k < 7; k++) pf[k] = __builtin_nontemporal_load(src + min(ti + 32 * k, bb - 1));
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
     if (blockIdx.x == 0 && t < NL) a.amax_key[t] = 0ull;   // the LM head that follows starts clean
-    int nu = a.uni[0];
-    nu = nu < 0 ? 0 : (nu > OXE_MAX_UNION ? OXE_MAX_UNION : nu);
     const bool exp_kq = a.exp_down_r.type != 8, sh_kq = a.sh_down_r.type != 8;
     if (t < DN_U) {
-        const int e = t < OXE_MAX_UNION ? (t < nu ? a.uni[1 + t] : -1) : 0;
-        s_e[t] = e < 0 ? 0 : (e < shp::NEXP ? e : shp::NEXP - 1);   // slots below compare the unclamped id
+        const int ue = t < OXE_MAX_UNION ? (t < nu ? a.uni[1 + t] : -1) : 0;
         for (int l = 0; l < NL; l++) {
             int j = -1;
             if (l < nl) {
                 if (t == OXE_MAX_UNION) j = shp::KUSED;
-                else if (e >= 0)
+                else if (ue >= 0)
                     for (int jj = 0; jj < shp::KUSED; jj++)
-                        if (a.route_ids[l * shp::KUSED + jj] == e) j = jj;
+                        if (a.route_ids[l * shp::KUSED + jj] == ue) j = jj;
             }
             s_slot[t][l] = j;
         }
     }
     if (t < NL * shp::KUSED) s_w[t / shp::KUSED][t % shp::KUSED] = t / shp::KUSED < nl ? a.route_w[t] : 0.0f;
     if (t < NL) s_sg[t] = t < nl ? a.sh_gate[t] : 0.0f;
-    // activations: activation row ar = l * DN_A + j (j = KUSED: the shared h)
-    if (exp_kq || sh_kq) {
-        for (int l = 0; l < NL; l++) {
-            if (exp_kq) stage_q8k(a.hk + (int64_t)l * shp::KUSED * DN_NB * Q8K_BYTES, shp::KUSED * DN_NB,
-                                  yh + l * DN_A * DN_NB * 2 * YH, yd + l * DN_A * DN_NB);
-            if (sh_kq) stage_q8k(a.hshk + (int64_t)l * DN_NB * Q8K_BYTES, DN_NB, yh + (l * DN_A + shp::KUSED) * DN_NB * 2 * YH,
-                                 yd + (l * DN_A + shp::KUSED) * DN_NB);
-        }
-    }
+    // activations: q8_K rows of every lane's slots, then of every lane's shared h; Q8_0 row l * DN_A + j (j = KUSED: the
+    // shared h)
+    constexpr int YSH = NL * shp::KUSED;   // first shared row
+    if (exp_kq) stage_q8k_all<DN_T, NL * shp::KUSED * DN_NB>(a.hk, yh, yd);
+    if (sh_kq) stage_q8k_all<DN_T, NL * DN_NB>(a.hshk, yh + YSH * DN_NB * 2 * YH, yd + YSH * DN_NB);
     if (!exp_kq || !sh_kq) {
-        for (int i = t; i < NL * DN_A * (shp::FF / 32); i += 256) {
-            const int ar = i / (shp::FF / 32), b = i % (shp::FF / 32), l = ar / DN_A, j = ar % DN_A;
+        for (int i = t; i < NL * DN_A * QB; i += DN_T) {
+            const int ar = i / QB, b = i % QB, l = ar / DN_A, j = ar % DN_A;
             const bool want = j < shp::KUSED ? !exp_kq : !sh_kq;
             if (want && l < nl) {
                 const float *src = j < shp::KUSED ? a.hexp + ((int64_t)l * shp::KUSED + j) * shp::FF + 32 * b
@@ -781,60 +834,59 @@ __global__ __launch_bounds__(256) void kq_down_kernel(const RunCtl *__restrict__
             }
         }
     }
-    __syncthreads();
-    // K-quant units, eight per pass: thread (unit u0 + t / 32, row t / 4 % 8, half block t % 4) forms
-    // its half block's integers for every lane with a slot there; threads t % 4 < NL then run lane
-    // t % 4's chain over the row's two blocks
-    static_assert(DN_R == 8, "thread mapping of the K-quant units");
-    {
-        const int p = t >> 5, rr = (t >> 2) & 7, hu = t & 3;
-        for (int u0 = 0; u0 < DN_U; u0 += 8) {
-            const int u = u0 + p;
-            const bool live = u < DN_U && (u == OXE_MAX_UNION ? sh_kq : (exp_kq && u < nu));
-            const RawW &W = u == OXE_MAX_UNION ? a.sh_down_r : a.exp_down_r;
-            const int type = W.type, rs = res_of(type), bb = kq_block_bytes(type);
-            const uint8_t *wr = live ? W.w + ((int64_t)s_e[u] * W.rows + row0 + rr) * raw_row_bytes(W) : nullptr;
-            if (live)
-                for (int l = 0; l < NL; l++) {
-                    const int j = s_slot[u][l];
-                    if (j >= 0)
-                        unit_rt<1>(type, wr + (hu >> 1) * bb, YView{yh + ((l * DN_A + j) * DN_NB * 2 + hu) * YH, 0}, hu & 1,
-                                   res + t * RS + l * rs);
-                }
-            __syncthreads();
-            if (live && hu < NL && s_slot[u][hu] >= 0) {
-                const int ar = hu * DN_A + s_slot[u][hu];
-                float acc = 0.0f;
-                for (int b = 0; b < DN_NB; b++) {
-                    const int *r0 = res + ((t & ~3) + 2 * b) * RS + hu * rs, *r1 = res + ((t & ~3) + 2 * b + 1) * RS + hu * rs;
-                    acc = chain_rt(type, acc, wr + b * bb, yd[ar * DN_NB + b], r0, r1);
-                }
-                s_dn[hu][s_slot[u][hu]][rr] = acc;
-            }
-            __syncthreads();
+    uint8_t *wl = s_wl[u < DN_U ? u : 0];
+    if (live) {
+        if (type == 8) {
+#pragma unroll
+            for (int k = 0; k < DN_LD - 1; k++) ((u32x4 *)wl)[ti + 32 * k] = pf[k];
+            ((u32x4 *)wl)[DN_R * shp::FF / 16 + (ti & 15)] = pf[DN_LD - 1];
+        } else {
+#pragma unroll
+            for (int k = 0; k < 7; k++) ((u32x4 *)wl)[min(ti + 32 * k, bb - 1)] = pf[k];   // clamped: same bytes
         }
     }
-    // Q8_0 units: one thread per (unit, lane, row), the block chain of the Q8_0 GEMV
-    for (int i = t; i < DN_U * NL * DN_R; i += 256) {
-        const int u = i / (NL * DN_R), l = (i / DN_R) % NL, rr = i % DN_R;
-        const bool sh = u == OXE_MAX_UNION;
-        if (sh ? sh_kq : (exp_kq || u >= nu)) continue;
-        const int j = s_slot[u][l];
-        if (j < 0) continue;
-        const int64_t row = row0 + rr;
-        const int8_t *wq = sh ? a.shexp_down.q + row * shp::FFSH : a.exp_down.q + ((int64_t)s_e[u] * shp::E + row) * shp::FF;
-        const uint16_t *wd = sh ? a.shexp_down.d + row * (shp::FFSH / 32)
-                                : a.exp_down.d + ((int64_t)s_e[u] * shp::E + row) * (shp::FF / 32);
-        const int ar = l * DN_A + j;
-        float acc = 0.0f;
-        for (int b = 0; b < shp::FF / 32; b++) {
-            int32_t s = 0;
+    __syncthreads();
+    // Integers of a unit: K-quant, thread (row ti / 4, half block ti % 4) for every lane with a slot there; Q8_0, block
+    // ti % 16 of rows ti / 16, + 2, ... Then threads ti % 4 < NL run lane ti % 4's chain over row ti / 4's blocks.
+    const int rr = ti >> 2, hu = ti & 3, rs = type != 8 ? res_of(type) : 0;
+    int *ru = res + (t & ~31) * RS;   // the unit's
+    if (live) {
+        for (int l = 0; l < NL; l++) {
+            const int j = s_slot[u][l];
+            if (j < 0) continue;
+            if (type != 8) {
+                const int ar = shu ? YSH + l : l * shp::KUSED + j;
+                unit_rt<1>(type, wl + (rr * DN_NB + (hu >> 1)) * bb, YView{yh + (ar * DN_NB * 2 + hu) * YH, 0}, hu & 1,
+                           res + t * RS + l * rs);
+            } else {
+                const int b = ti & 15;
+                for (int r = ti >> 4; r < DN_R; r += 2) {
+                    const u32x4 *wp = (const u32x4 *)(wl + r * shp::FF + 32 * b), *xp = (const u32x4 *)&s_q[l * DN_A + j][32 * b];
+                    int32_t s = 0;
 #pragma unroll
-            for (int k = 0; k < 8; k++)
-                s = dot4(*(const uint32_t *)(wq + 32 * b + 4 * k), *(const uint32_t *)&s_q[ar][32 * b + 4 * k], s);
-            acc = __builtin_fmaf((float)s, h2f(s_d[ar][b]) * h2f(wd[b]), acc);
+                    for (int k = 0; k < 8; k++) s = dot4(wp[k >> 2][k & 3], xp[k >> 2][k & 3], s);
+                    ru[(l * DN_R + r) * QB + b] = s;
+                }
+            }
         }
-        s_dn[l][j][rr] = acc;
+    }
+    __syncthreads();
+    if (live && hu < NL && s_slot[u][hu] >= 0) {
+        const int j = s_slot[u][hu];
+        float acc = 0.0f;
+        if (type != 8) {
+            const int ar = shu ? YSH + hu : hu * shp::KUSED + j;
+            for (int b = 0; b < DN_NB; b++) {
+                const int *r0 = res + ((t & ~3) + 2 * b) * RS + hu * rs, *r1 = res + ((t & ~3) + 2 * b + 1) * RS + hu * rs;
+                acc = chain_rt(type, acc, wl + (rr * DN_NB + b) * bb, yd[ar * DN_NB + b], r0, r1);
+            }
+        } else {
+            const uint16_t *wd = (const uint16_t *)(wl + DN_R * shp::FF) + rr * QB, *xd = s_d[hu * DN_A + j];
+            const int *is = ru + (hu * DN_R + rr) * QB;
+#pragma unroll
+            for (int b = 0; b < QB; b++) acc = __builtin_fmaf((float)is[b], h2f(xd[b]) * h2f(wd[b]), acc);
+        }
+        s_dn[hu][j][rr] = acc;
     }
     __syncthreads();
     if (t < NL * DN_R) {
@@ -994,7 +1046,11 @@ int launch_kq_moe(const RunCtl *ctl, const ModelRt &m, const LayerW &w, const Ac
         a.do_exp = exp_gu;
         a.do_sh = sh_gu;
         a.stats = b.counters + CNT_UNI_SUM;
-        hipLaunchKernelGGL(kq::kq_gu_kernel<OXE_NL>, dim3((OXE_MAX_UNION + 1) * (shp::FF / kq::GU_R)), dim3(256), 0, st, ctl, a);
+        // a tile's gate and up rows in LDS, of whichever unit is larger
+        const int64_t le = exp_gu ? raw_row_bytes(a.gate) + raw_row_bytes(a.up) : 0;
+        const int64_t ls = sh_gu ? raw_row_bytes(a.sh_gate) + raw_row_bytes(a.sh_up) : 0;
+        hipLaunchKernelGGL(kq::kq_gu_kernel<OXE_NL>, dim3((OXE_MAX_UNION + 1) * (shp::FF / kq::GU_R)), dim3(256),
+                           (size_t)(kq::GU_R * std::max(le, ls)), st, ctl, a);
     }
     {
         // h of the routed slots and of the shared expert, for whichever down matrices are K-quants
@@ -1020,7 +1076,7 @@ int launch_kq_moe(const RunCtl *ctl, const ModelRt &m, const LayerW &w, const Ac
     d.x1 = b.x1;
     d.x2 = b.x2;
     d.amax_key = b.amax_key;
-    hipLaunchKernelGGL(kq::kq_down_kernel<OXE_NL>, dim3(shp::E / kq::DN_R), dim3(256), 0, st, ctl, d);
+    hipLaunchKernelGGL(kq::kq_down_kernel<OXE_NL>, dim3(shp::E / kq::DN_R), dim3(kq::DN_T), 0, st, ctl, d);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
