@@ -62,20 +62,6 @@ __global__ __launch_bounds__(256) void quant_q8_K_kernel(const float *__restrict
     q8K_block(x + b * QK, threadIdx.x & 63, y + b * Q8K_BYTES);
 }
 
-// two buffers' blocks in one launch: blocks b < n0 of x0 into y0, then n1 of x1 into y1
-__global__ __launch_bounds__(256) void quant_q8_K_two_kernel(const float *__restrict__ x0, int64_t n0,
-                                                             uint8_t *__restrict__ y0, const float *__restrict__ x1,
-                                                             int64_t n1, uint8_t *__restrict__ y1) {
-    int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (b >= n0 + n1) return;
-    if (b < n0) {
-        q8K_block(x0 + b * QK, threadIdx.x & 63, y0 + b * Q8K_BYTES);
-    } else {
-        b -= n0;
-        q8K_block(x1 + b * QK, threadIdx.x & 63, y1 + b * Q8K_BYTES);
-    }
-}
-
 // the q8_K blocks of a workgroup's [NL][E] rows held in LDS (256 threads: wave w takes blocks w,
 // w + 4, ...), after the barrier that completes the rows
 template <int NL>
@@ -565,35 +551,29 @@ OXE_DEV float chain_rt(int type, float acc, const uint8_t *wb, float dx, const i
 OXE_DEV int res_of(int type) { return type == 12 ? BT<4>::R : type == 13 ? BT<5>::R : 1; }
 constexpr int RES_MAX = 6;
 
-// nblk q8_K blocks (292 bytes each, from y) into LDS as halves (YH words apart) and scales
-OXE_DEV void stage_q8k(const uint8_t *y, int nblk, uint32_t *yh, float *yd) {
-    for (int i = threadIdx.x; i < nblk * 2 * 36; i += blockDim.x) {
-        const int wd = i % 36, hb = i / 36, h = hb & 1;
-        const uint32_t *src = (const uint32_t *)(y + (int64_t)(hb >> 1) * Q8K_BYTES);
-        yh[hb * YH + wd] = wd < 32 ? src[1 + 32 * h + wd] : src[65 + 4 * h + (wd - 32)];
-    }
-    for (int i = threadIdx.x; i < nblk; i += blockDim.x) yd[i] = *(const float *)(y + (int64_t)i * Q8K_BYTES);
-}
-
-// the same with a workgroup of T threads and NBLK blocks, every load in flight at once
-template <int T, int NBLK>
-OXE_DEV void stage_q8k_all(const uint8_t *y, uint32_t *yh, float *yd) {
-    constexpr int N = NBLK * 2 * 36, I = (N + T - 1) / T;
-    static_assert(NBLK <= T, "one scale per thread");
-    uint32_t v[I];
+// q8_K of NBLK blocks of floats by a workgroup of W waves into LDS, as halves (YH words apart) and scales, every load in
+// flight at once. Each workgroup of gate / up and of down quantises what it reads, 1.5 us more of a launch each (the
+// launches that did it before them took 4.3 and 4.5)
+template <int W, int NBLK>
+OXE_DEV void quant_q8k_lds(const float *x, uint32_t *yh, float *yd) {
+    constexpr int I = (NBLK + W - 1) / W;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float4 f[I];
+#pragma unroll
+    for (int k = 0; k < I; k++) f[k] = *(const float4 *)(x + min(w + W * k, NBLK - 1) * QK + 4 * lane);
 #pragma unroll
     for (int k = 0; k < I; k++) {
-        const int i = min((int)threadIdx.x + T * k, N - 1), wd = i % 36, hb = i / 36, h = hb & 1;
-        const uint32_t *src = (const uint32_t *)(y + (int64_t)(hb >> 1) * Q8K_BYTES);
-        v[k] = wd < 32 ? src[1 + 32 * h + wd] : src[65 + 4 * h + (wd - 32)];
+        const int b = w + W * k;
+        if (b >= NBLK) break;   // wave-uniform
+        const float v[4] = {f[k].x, f[k].y, f[k].z, f[k].w};
+        int q[4];
+        const float d = q8K_codes(v, lane, q);
+        const int s = sum16(q);
+        uint32_t *y = yh + (2 * b + (lane >> 5)) * YH;
+        y[lane & 31] = pack4(q);
+        if ((lane & 3) == 0) ((int16_t *)(y + 32))[(lane >> 2) & 7] = (int16_t)s;
+        if (lane == 0) yd[b] = d;
     }
-    const float d = *(const float *)(y + (int64_t)min((int)threadIdx.x, NBLK - 1) * Q8K_BYTES);
-#pragma unroll
-    for (int k = 0; k < I; k++) {
-        const int i = min((int)threadIdx.x + T * k, N - 1);
-        yh[i / 36 * YH + i % 36] = v[k];
-    }
-    if (threadIdx.x < NBLK) yd[threadIdx.x] = d;
 }
 
 OXE_DEV uint32_t ordered_bits(float f) {
@@ -656,9 +636,9 @@ __global__ __launch_bounds__(256) void ba_f32_kernel(const RunCtl *__restrict__ 
 // (ggml_v_silu, as swiglu) for every lane that routed to the expert (the shared expert: every lane).
 // A tile's rows are one run of bytes per matrix: they come as whole lines, before the activations, and are read from
 // LDS (each thread reading its half block from global memory after the activations, 64 threads 72 bytes apart: 18.4 us a
-// launch with Q4_K experts of two lanes, 14.2 so). Bound by the latency of one round of workgroups.
+// launch with Q4_K experts of two lanes, 14.2 so, both after a launch that quantised xn). Bound by the latency of one round of workgroups.
 struct KqGuArgs {
-    const uint8_t *xk;          // [NL][E / 256] q8_K blocks of xn
+    const float *xn;            // [NL][E]
     RawW gate, up, sh_gate, sh_up;
     const int32_t *uni, *route_ids;
     float *hexp;                // [NL][KUSED][FF]
@@ -700,7 +680,7 @@ __global__ __launch_bounds__(256) void kq_gu_kernel(const RunCtl *__restrict__ c
 #pragma unroll
     for (int k = 0; k < GU_LD; k++) pf[k] = __builtin_nontemporal_load(src + min((t & 127) + 128 * k, n16 - 1));
     __builtin_amdgcn_sched_barrier(0);   // the weights before the activations
-    stage_q8k_all<256, NL * GU_NB>(a.xk, yh, yd);
+    quant_q8k_lds<4, NL * GU_NB>(a.xn, yh, yd);
     int slot = -1;
     if (which == 0 && hu < NL && hu < nl && !sh)
 #pragma unroll
@@ -741,12 +721,12 @@ __global__ __launch_bounds__(256) void kq_gu_kernel(const RunCtl *__restrict__ c
 // 32 threads per unit, every unit at once: a unit's 8 rows are one run of bytes, requested as whole lines before
 // anything else and read from LDS, so the launch waits for memory once (256 workgroups, one per CU, whose 125 KB
 // of LDS and registers nothing else wants). Eight units a pass from global memory, the Q8_0 unit's blocks by one
-// thread per row: 17.2 us a launch with Q5_K experts and a Q8_0 shared matrix, two lanes; 8.8 so.
+// thread per row: 17.2 us a launch with Q5_K experts and a Q8_0 shared matrix, two lanes; 8.8 so, both after
+// a launch that quantised h.
 struct KqDownArgs {
     const int32_t *uni, *route_ids;
     const float *route_w, *sh_gate;
-    const float *hexp, *hsh;        // f32 h (Q8_0 matrices quantise it here)
-    const uint8_t *hk, *hshk;       // q8_K blocks of h (K-quant matrices)
+    const float *hexp, *hsh;        // f32 h, quantised here
     Q8W exp_down, shexp_down;
     RawW exp_down_r, sh_down_r;
     const float *x1;
@@ -821,8 +801,8 @@ __global__ __launch_bounds__(DN_T) void kq_down_kernel(const RunCtl *__restrict_
     // activations: q8_K rows of every lane's slots, then of every lane's shared h; Q8_0 row l * DN_A + j (j = KUSED: the
     // shared h)
     constexpr int YSH = NL * shp::KUSED;   // first shared row
-    if (exp_kq) stage_q8k_all<DN_T, NL * shp::KUSED * DN_NB>(a.hk, yh, yd);
-    if (sh_kq) stage_q8k_all<DN_T, NL * DN_NB>(a.hshk, yh + YSH * DN_NB * 2 * YH, yd + YSH * DN_NB);
+    if (exp_kq) quant_q8k_lds<DN_T / 64, NL * shp::KUSED * DN_NB>(a.hexp, yh, yd);
+    if (sh_kq) quant_q8k_lds<DN_T / 64, NL * DN_NB>(a.hsh, yh + YSH * DN_NB * 2 * YH, yd + YSH * DN_NB);
     if (!exp_kq || !sh_kq) {
         for (int i = t; i < NL * DN_A * QB; i += DN_T) {
             const int ar = i / QB, b = i % QB, l = ar / DN_A, j = ar % DN_A;
@@ -1030,11 +1010,10 @@ static void quant_k(const float *x, int64_t nblk, uint8_t *y, hipStream_t st) {
 int launch_kq_moe(const RunCtl *ctl, const ModelRt &m, const LayerW &w, const ActBufs &b, hipStream_t st) {
     (void)m;
     const bool exp_gu = w.exp_gate_r.type != 8, sh_gu = w.sh_gate_r.type != 8;
-    if (exp_gu || sh_gu) quant_k(b.xn, (int64_t)OXE_NL * shp::E / kq::QK, b.xk, st);
     if (!exp_gu) launch_experts(ctl, w, b, st);
     if (exp_gu || sh_gu) {
         kq::KqGuArgs a{};
-        a.xk = b.xk;
+        a.xn = b.xn;
         a.gate = w.exp_gate_r;
         a.up = w.exp_up_r;
         a.sh_gate = w.sh_gate_r;
@@ -1052,14 +1031,6 @@ int launch_kq_moe(const RunCtl *ctl, const ModelRt &m, const LayerW &w, const Ac
         hipLaunchKernelGGL(kq::kq_gu_kernel<OXE_NL>, dim3((OXE_MAX_UNION + 1) * (shp::FF / kq::GU_R)), dim3(256),
                            (size_t)(kq::GU_R * std::max(le, ls)), st, ctl, a);
     }
-    {
-        // h of the routed slots and of the shared expert, for whichever down matrices are K-quants
-        const int64_t ne = w.exp_down_r.type != 8 ? (int64_t)OXE_NL * shp::KUSED * shp::FF / kq::QK : 0;
-        const int64_t ns = w.sh_down_r.type != 8 ? (int64_t)OXE_NL * shp::FFSH / kq::QK : 0;
-        if (ne + ns > 0)
-            hipLaunchKernelGGL(kq::quant_q8_K_two_kernel, dim3((unsigned)((ne + ns + 3) / 4)), dim3(256), 0, st, b.hexp, ne,
-                               b.hk, b.hsh, ns, b.hshk);
-    }
     kq::KqDownArgs d{};
     d.uni = b.uni;
     d.route_ids = b.route_ids;
@@ -1067,8 +1038,6 @@ int launch_kq_moe(const RunCtl *ctl, const ModelRt &m, const LayerW &w, const Ac
     d.sh_gate = b.sh_gate;
     d.hexp = b.hexp;
     d.hsh = b.hsh;
-    d.hk = b.hk;
-    d.hshk = b.hshk;
     d.exp_down = w.exp_down;
     d.shexp_down = w.shexp_down;
     d.exp_down_r = w.exp_down_r;

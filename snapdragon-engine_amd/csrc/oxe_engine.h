@@ -163,8 +163,6 @@ struct ActBufs {
     float *logits;        // [NL][n_vocab] (optional)
     unsigned long long *amax_key;  // [NL] packed argmax keys
     uint8_t *xk;          // q8_K blocks of xn [NL][n_embd / 256] (K-quant matrices)
-    uint8_t *hk;          // q8_K blocks of hexp [NL][k_used][ff_exp / 256]
-    uint8_t *hshk;        // q8_K blocks of hsh [NL][ff_shexp / 256]
     float *o32;           // the mixer's gated outputs in f32 [NL][4096] (a K-quant output projection)
     uint8_t *ok;          // their q8_K blocks [NL][4096 / 256]
     float *emb;           // the lanes' embedded tokens [NL][n_embd] (a K-quant token embedding)

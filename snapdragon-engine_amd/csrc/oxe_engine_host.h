@@ -392,8 +392,6 @@ struct Engine {
         b.logits = alloc<float>((size_t)OXE_NL * d.n_vocab);
         b.amax_key = alloc<unsigned long long>(OXE_NL);
         b.xk = alloc<uint8_t>((size_t)OXE_NL * (E / 256) * 292);
-        b.hk = alloc<uint8_t>((size_t)OXE_NL * KUSED * (FF / 256) * 292);
-        b.hshk = alloc<uint8_t>((size_t)OXE_NL * (FFSH / 256) * 292);
         if (kq) {
             b.o32 = alloc<float>(OXE_NL * MIX_W);
             b.ok = alloc<uint8_t>((size_t)OXE_NL * (MIX_W / 256) * 292);
