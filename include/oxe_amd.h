@@ -245,7 +245,7 @@ OXE_API int oxe_gguf_model_desc(const oxe_gguf *g, oxe_model_desc *out);
  * which oxe_engine_create_from_gguf reads from the file; into an engine created for Q8_0 they are
  * refused by name (-1), as is any other tensor type. An engine with such matrices runs its runs per
  * phase (oxe_engine_set_fused(e, 1) returns -1: the fused run kernel reads Q8_0 matrices only) and
- * its batched prefill as decode runs of two positions (the same state and h_nextn). */
+ * its batched prefill of one or two positions as a decode run (the same state and h_nextn). */
 OXE_API int oxe_engine_load_gguf(oxe_engine *e, const oxe_gguf *g);
 /* oxe_engine_load_gguf without any device allocation: no counterpart in the reference; for callers
  * that cannot allocate device memory (code under HIP graph capture, serving loops, harnesses that
