@@ -175,6 +175,9 @@ OXE_API int64_t oxe_engine_kv_row_bytes(const oxe_engine *e);
 OXE_API int oxe_engine_write_kv_rows(oxe_engine *e, int a, int b, void *host, int64_t cap);
 OXE_API int oxe_engine_read_kv_rows(oxe_engine *e, int a, int b, const void *host, int64_t nbytes);
 OXE_API int64_t oxe_engine_device_bytes(const oxe_engine *e);
+/* Device memory the engine may hold from now on (max <= 0: no limit): a buffer that it would allocate
+ * past max is refused as when the device is out of memory. Diagnostic (no counterpart in the reference). */
+OXE_API void oxe_engine_limit_bytes(oxe_engine *e, int64_t max);
 /* Run mode (no counterpart in the reference, whose runs are thread-team phases): 1 = every run
  * as one persistent launch of the fused run kernel (the default where the device has exactly 256
  * CUs), 0 = one launch per phase. Both compute the same bits. -1 when 1 is not available. */
@@ -245,7 +248,8 @@ OXE_API int oxe_gguf_model_desc(const oxe_gguf *g, oxe_model_desc *out);
  * which oxe_engine_create_from_gguf reads from the file; into an engine created for Q8_0 they are
  * refused by name (-1), as is any other tensor type. An engine with such matrices runs its runs per
  * phase (oxe_engine_set_fused(e, 1) returns -1: the fused run kernel reads Q8_0 matrices only) and
- * its batched prefill of one or two positions as a decode run (the same state and h_nextn). */
+ * its batched prefill as decode runs of two positions where there are at most two, or where the
+ * device is out of memory for the batched pass (the same state and h_nextn). */
 OXE_API int oxe_engine_load_gguf(oxe_engine *e, const oxe_gguf *g);
 /* oxe_engine_load_gguf without any device allocation: no counterpart in the reference; for callers
  * that cannot allocate device memory (code under HIP graph capture, serving loops, harnesses that

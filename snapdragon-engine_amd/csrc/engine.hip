@@ -302,6 +302,7 @@ int oxe_engine_set_router(oxe_engine *e, int layer, int row0, int nrows, const f
 }
 
 int64_t oxe_engine_device_bytes(const oxe_engine *e) { return (int64_t)((const Engine *)e)->bytes; }
+void oxe_engine_limit_bytes(oxe_engine *e, int64_t max) { ((Engine *)e)->bytes_max = max > 0 ? (size_t)max : SIZE_MAX; }
 
 // Engine::state_bytes (engine.rs:1570-1576): K and V^T of the positions < pos of every attention
 // layer (the MTP layer's included), f16, then the current slot's conv and delta-net state, f32.

@@ -924,7 +924,7 @@ int Engine::pf_alloc(int T) {
         }
         pfb.cap = T;
     } catch (...) {
-        set_err("out of device memory for the prefill buffers");
+        if (!kq) set_err("out of device memory for the prefill buffers");   // a typed engine has its decode runs
         return -3;
     }
     return 0;
@@ -1158,32 +1158,34 @@ int Engine::pf_chunk(const uint32_t *toks, int T, float *h_out) {
     return 0;
 }
 
+// the prompt as decode runs of two positions (every position's state and h_nextn are the batched pass's)
+int Engine::prefill_runs(const uint32_t *toks, int n, uint32_t *next, float *h_all) {
+    uint32_t g[OXE_NL] = {};
+    for (int c0 = 0; c0 < n; c0 += OXE_NL) {
+        const int c = std::min(OXE_NL, n - c0);
+        int rc = verify(toks + c0, c, g);
+        if (!rc) rc = commit(c);
+        if (rc) return rc;
+        for (int i = 0; i < c && h_all; i++)
+            if ((rc = hidden_host(i, h_all + (size_t)(c0 + i) * E))) return rc;
+    }
+    const int last = (n - 1) % OXE_NL;   // the last token's lane: its row is lane 0's after a prefill
+    if (last) {
+        if (hipMemcpyAsync(b.logits, b.logits + (size_t)last * d.n_vocab, (size_t)d.n_vocab * 4, hipMemcpyDeviceToDevice,
+                           st) != hipSuccess ||
+            hipMemcpyAsync(b.hid, b.hid + (size_t)last * E, (size_t)E * 4, hipMemcpyDeviceToDevice, st) != hipSuccess ||
+            hipStreamSynchronize(st) != hipSuccess)
+            return -2;
+    }
+    if (next) *next = g[last];
+    return 0;
+}
+
 int Engine::prefill(const uint32_t *toks, int n, uint32_t *next, float *h_all) {
     if (n < 1 || pos + n > m.n_ctx || !toks_ok(toks, n)) return -1;
-    if (kq && n <= PF_KQ_RUNS) {
-        // a few positions of a model with K-quant / F32 matrices: decode runs of two positions (every
-        // position's state and h_nextn are the batched pass's)
-        uint32_t g[OXE_NL] = {};
-        for (int c0 = 0; c0 < n; c0 += OXE_NL) {
-            const int c = std::min(OXE_NL, n - c0);
-            int rc = verify(toks + c0, c, g);
-            if (!rc) rc = commit(c);
-            if (rc) return rc;
-            for (int i = 0; i < c && h_all; i++)
-                if ((rc = hidden_host(i, h_all + (size_t)(c0 + i) * E))) return rc;
-        }
-        const int last = (n - 1) % OXE_NL;   // the last token's lane: its row is lane 0's after a prefill
-        if (last) {
-            if (hipMemcpyAsync(b.logits, b.logits + (size_t)last * d.n_vocab, (size_t)d.n_vocab * 4, hipMemcpyDeviceToDevice,
-                               st) != hipSuccess ||
-                hipMemcpyAsync(b.hid, b.hid + (size_t)last * E, (size_t)E * 4, hipMemcpyDeviceToDevice, st) != hipSuccess ||
-                hipStreamSynchronize(st) != hipSuccess)
-                return -2;
-        }
-        if (next) *next = g[last];
-        return 0;
-    }
+    if (kq && n <= PF_KQ_RUNS) return prefill_runs(toks, n, next, h_all);
     int rc = pf_alloc(std::min(n, PF_CHUNK));
+    if (rc && kq) return prefill_runs(toks, n, next, h_all);   // no memory for a batched pass: the runs need none
     if (rc) return rc;
     pend_n = 0;
     for (int c0 = 0; c0 < n; c0 += PF_CHUNK) {
@@ -1213,6 +1215,11 @@ int Engine::seed_batched(const uint32_t *toks, int n, int pos0, const float *hs)
     const LayerW &w = L[d.n_layer];
     const bool kemb = m.tok_embd_r.type != 8, kproj = w.kq_proj();
     int rc = pf_alloc(std::min(n, PF_CHUNK));
+    if (rc && kq) {   // no memory for a batched pass: seeding runs of two pairs (every pair's rows depend on that pair only)
+        for (int c0 = 0; c0 < n; c0 += OXE_NL)
+            if ((rc = mtp_seed(toks + c0, std::min(OXE_NL, n - c0), pos0 + c0, hs + (size_t)c0 * E))) return rc;
+        return 0;
+    }
     if (rc) return rc;
     uint16_t *kcl = m.kcache + (int64_t)w.index * NKV * m.n_ctx * HD;
     uint16_t *vtl = m.vcache + (int64_t)w.index * NKV * HD * m.n_ctx;

@@ -92,7 +92,7 @@ struct Engine {
     // commit kernel or by dev_begin
     RunCtl *ctl_draft = nullptr;
     std::vector<void *> allocs;
-    size_t bytes = 0;
+    size_t bytes = 0, bytes_max = SIZE_MAX;   // device memory held, and its limit (oxe_engine_limit_bytes)
     // host mirror of the engine position (host-driven API)
     int pos = 0, cur = 0;
     int pend_pos0 = 0, pend_cur = 0, pend_n = 0, pend_done = 0;
@@ -128,6 +128,7 @@ struct Engine {
     int pf_alloc(int T);
     int pf_attn_lds(int kv_cap);
     int pf_chunk(const uint32_t *toks, int T, float *h_out);
+    int prefill_runs(const uint32_t *toks, int n, uint32_t *next, float *h_all);
     int prefill(const uint32_t *toks, int n, uint32_t *next, float *h_all);
     int seed_batched(const uint32_t *toks, int n, int pos0, const float *hs);
     // weights from a GGUF file (k_load.hip): through a staging buffer allocated for the call, or
@@ -209,7 +210,11 @@ struct Engine {
     template <class T>
     T *alloc(size_t n) {
         void *p = nullptr;
-        if (hipMalloc(&p, n * sizeof(T) + 64) != hipSuccess) throw std::runtime_error("hipMalloc failed");
+        if (bytes > bytes_max || n * sizeof(T) > bytes_max - bytes) throw std::runtime_error("device memory limit reached");
+        if (hipMalloc(&p, n * sizeof(T) + 64) != hipSuccess) {
+            (void)hipGetLastError();   // not the next launch check's
+            throw std::runtime_error("hipMalloc failed");
+        }
         allocs.push_back(p);
         bytes += n * sizeof(T);
         return (T *)p;

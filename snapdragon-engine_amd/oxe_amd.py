@@ -269,6 +269,7 @@ def _engine_sigs(L):
         "oxe_engine_set_pos": (i32, [vp, i32]),
         "oxe_engine_set_router": (i32, [vp, i32, i32, i32, f32p]),
         "oxe_engine_device_bytes": (i64, [vp]),
+        "oxe_engine_limit_bytes": (None, [vp, i64]),
         "oxe_engine_state_bytes": (i64, [vp]),
         "oxe_engine_write_state": (i32, [vp, vp, i64]),
         "oxe_engine_read_state": (i32, [vp, vp, i64, i32]),
