@@ -125,7 +125,10 @@ struct Engine {
     int nkeys() const { return fused ? fz_grid : 1; }
     // batched prefill (k_prefill.hip)
     PfBufs pfb{};
+    void *pf_mem = nullptr;   // its buffers, one allocation, given back when a longer prompt needs a larger one
+    size_t pf_bytes = 0;
     int pf_alloc(int T);
+    void pf_free();
     int pf_attn_lds(int kv_cap);
     int pf_chunk(const uint32_t *toks, int T, float *h_out);
     int prefill_runs(const uint32_t *toks, int n, uint32_t *next, float *h_all);
@@ -232,6 +235,7 @@ struct Engine {
         if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
         (void)hipStreamSynchronize(st);
         for (void *p : allocs) (void)hipFree(p);
+        if (pf_mem) (void)hipFree(pf_mem);
         if (st && own_stream) (void)hipStreamDestroy(st);
     }
 

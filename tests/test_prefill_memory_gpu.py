@@ -1,4 +1,4 @@
-"""Device memory of the batched prefill: what happens when its buffers do not fit. The engine's own limit
+"""Device memory of the batched prefill: what its buffers hold as prompts grow, and what happens when they do not fit. The engine's own limit
 (oxe_engine_limit_bytes) stands in for a full device."""
 import numpy as np
 import pytest
@@ -68,5 +68,40 @@ def test_q8_0_prefill_without_memory_is_refused():
     limit(a, 0)
     assert a.prefill(toks) == b.prefill(toks)
     assert_same_state(a, b, d, "after the limit went")
+    for e in (a, b):
+        e.close()
+
+
+@pytest.mark.parametrize("types", [None, "every type"])
+def test_growing_prompts_hold_one_set_of_buffers(types):
+    """a longer prompt's buffers replace the shorter one's; a set that does not fit leaves none behind"""
+    import oxe_amd as A
+    d = O.desc_small()
+    ty = types and model_types(types)
+    a, b = (A.Engine(d, seed=7, n_ctx=512, types=ty) for _ in range(2))
+    toks = prompt(d, 240)
+    bare = held(b)
+    b.prefill(toks[:100])
+    for lo, hi in ((0, 20), (20, 60), (60, 140), (140, 240)):   # 20, 40, 80, 100 tokens
+        print(f"prefill {types} {lo}..{hi}", flush=True)
+        x = a.prefill(toks[lo:hi])
+    assert held(a) == held(b) > bare
+    b.prefill(toks[100:190])
+    assert x == b.prefill(toks[190:])
+    assert held(a) == held(b)
+    assert_same_state(a, b, d, "grown against one size", main_only=True)
+    limit(a, held(a))
+    print(f"prefill {types} at the limit", flush=True)
+    if ty:
+        assert a.prefill(toks[:120]) == b.prefill(toks[:120])
+    else:
+        with pytest.raises(RuntimeError, match="out of device memory"):
+            a.prefill(toks[:120])
+        b.prefill(toks[:120])
+        for t in toks[:120]:
+            a.step(t)
+    assert held(a) == bare
+    assert a.prefill(toks[:50]) == b.prefill(toks[:50])   # what fits is taken again
+    assert held(a) > bare
     for e in (a, b):
         e.close()
