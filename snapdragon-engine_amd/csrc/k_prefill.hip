@@ -927,7 +927,6 @@ int Engine::pf_alloc(int T) {
         take(pfb.hq, nr * FF);
         take(pfb.hd, nr * (FF / 32));
         take(pfb.dout, nr * E);
-        take(pfb.sh, (size_t)T * E);
         take(pfb.tok, (size_t)T);
         if (kq) {
             auto act = [&](size_t rows, size_t k) {
@@ -1136,6 +1135,7 @@ int Engine::pf_chunk(const uint32_t *toks, int T, float *h_out) {
             return kq_pf_swiglu_q8_0(pfb.gu, split, rows, pfb.hq, pfb.hd, st);
         };
         KqAct h{};
+        float *const sh = pfb.dout + (int64_t)np * E;   // the shared expert's rows, after the pairs'
         // routed experts: pairs grouped by expert, 64-pair tiles built on the device. With Q8_0 matrices throughout the
         // shared expert is one more group: its rows fill the experts' launches and need none of their own
         const bool join = !kegu && !ksgu && !kedn && !ksdn;
@@ -1146,24 +1146,24 @@ int Engine::pf_chunk(const uint32_t *toks, int T, float *h_out) {
             if ((rc = kq_pf_swiglu_q8_0(pfb.gu, false, np + T, pfb.hq, pfb.hd, st))) return rc;
             if ((rc = grouped(w.exp_down, E, FF, pfb.hq, pfb.hd, nullptr, pfb.dout, &w.shexp_down))) return rc;
         } else {
-        // shared expert over all tokens
-        if (ksgu) rc = kgemm(sgu, 2, E, xa, pfb.gu, 2 * FFSH, nullptr, T, nullptr, false);
-        else rc = gemm(w.shexp_gu, pfb.xq, pfb.xd, E, pfb.gu, 2 * FFSH, nullptr, T);
-        if (rc) return rc;
-        if ((rc = swiglu(ksgu, sdn, T, h))) return rc;
-        if (ksdn) rc = kgemm(sdn, 1, FFSH, h, pfb.sh, E, nullptr, T, nullptr, false);
-        else rc = gemm(w.shexp_down, pfb.hq, pfb.hd, FFSH, pfb.sh, E, nullptr, T);
-        if (rc) return rc;
-        if (kegu) rc = kgemm(egu, 2, E, xa, pfb.gu, 2 * FF, nullptr, T, pfb.ptok, true);
-        else rc = grouped(w.exp_gu, 2 * FF, E, pfb.xq, pfb.xd, pfb.ptok, pfb.gu, nullptr);
-        if (rc) return rc;
-        if ((rc = swiglu(kegu, edn, np, h))) return rc;
-        if (kedn) rc = kgemm(edn, 1, FF, h, pfb.dout, E, nullptr, np, nullptr, true);
-        else rc = grouped(w.exp_down, E, FF, pfb.hq, pfb.hd, nullptr, pfb.dout, nullptr);
-        if (rc) return rc;
+            // shared expert over all tokens
+            if (ksgu) rc = kgemm(sgu, 2, E, xa, pfb.gu, 2 * FFSH, nullptr, T, nullptr, false);
+            else rc = gemm(w.shexp_gu, pfb.xq, pfb.xd, E, pfb.gu, 2 * FFSH, nullptr, T);
+            if (rc) return rc;
+            if ((rc = swiglu(ksgu, sdn, T, h))) return rc;
+            if (ksdn) rc = kgemm(sdn, 1, FFSH, h, sh, E, nullptr, T, nullptr, false);
+            else rc = gemm(w.shexp_down, pfb.hq, pfb.hd, FFSH, sh, E, nullptr, T);
+            if (rc) return rc;
+            if (kegu) rc = kgemm(egu, 2, E, xa, pfb.gu, 2 * FF, nullptr, T, pfb.ptok, true);
+            else rc = grouped(w.exp_gu, 2 * FF, E, pfb.xq, pfb.xd, pfb.ptok, pfb.gu, nullptr);
+            if (rc) return rc;
+            if ((rc = swiglu(kegu, edn, np, h))) return rc;
+            if (kedn) rc = kgemm(edn, 1, FF, h, pfb.dout, E, nullptr, np, nullptr, true);
+            else rc = grouped(w.exp_down, E, FF, pfb.hq, pfb.hd, nullptr, pfb.dout, nullptr);
+            if (rc) return rc;
         }
         hipLaunchKernelGGL(combine_kernel, dim3((unsigned)(((int64_t)T * E + 255) / 256)), dim3(256), 0, st, pfb.dout,
-                           pfb.pair_of, pfb.wts, join ? pfb.dout + (int64_t)np * E : pfb.sh, pfb.sg, pfb.x1, pfb.x, T);
+                           pfb.pair_of, pfb.wts, sh, pfb.sg, pfb.x1, pfb.x, T);
         if (hipGetLastError() != hipSuccess) return -2;
     }
     // h_nextn of every token (output norm of x2), the LM head of the last token

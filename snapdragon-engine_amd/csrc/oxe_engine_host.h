@@ -58,7 +58,7 @@ struct MtpDriverHost {
 // Buffers of the batched prefill, [T][...] for up to cap tokens (allocated on first use)
 struct PfBufs {
     int cap = 0, max_tiles = 0, attn_lds = 0, attn_lds_gqa = 0;
-    float *x, *x1, *xn, *hin, *proj, *cy, *gg, *gb, *o, *lg, *sg, *wts, *gu, *dout, *sh;
+    float *x, *x1, *xn, *hin, *proj, *cy, *gg, *gb, *o, *lg, *sg, *wts, *gu, *dout;
     int8_t *xq, *oq, *hq;
     uint16_t *xd, *od, *qh, *hd;
     int32_t *ids, *mo, *ptok, *pair_of;
