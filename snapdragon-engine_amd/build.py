@@ -3,7 +3,7 @@
 Flags that the parity contract depends on:
   -ffp-contract=off                           no implicit multiply-add fusion (every fma is explicit)
   -fhip-fp32-correctly-rounded-divide-sqrt    IEEE f32 division and sqrt (the reference's libm/CPU ones)
-  -Xclang -target-feature -Xclang -packed-fp32-ops   no packed-f32 instructions (unreliable on this pool)
+  -Xclang -target-feature -Xclang -packed-fp32-ops   no packed-f32 instructions (some forms give wrong results)
 """
 import os
 import subprocess

@@ -304,8 +304,6 @@ OXE_DEV SegRef seg_ref(const KqSegs &S, int64_t g) {
     return r;
 }
 
-// one group of 4 rows (g may be past the end: then nothing is written): its prefetched bytes (pf)
-// and the rest to LDS, pf refilled with group g_next, then the units and the chains
 // LDS accesses of this wave before it come before those after it (wave-private regions: no barrier)
 OXE_DEV void wave_fence() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -322,6 +320,8 @@ __host__ __device__ inline int vl_wave_lds(int bb, int rr, int nb, int nl) {
     return align16(GR * nb * bb) + align16(64 * ((nl * rr) | 1) * 4);
 }
 
+// one group of 4 rows (g may be past the end: then nothing is written): its prefetched bytes (pf)
+// and the rest to LDS, pf refilled with group g_next, then the units and the chains
 template <int TY, int NL, int PF, int NW>
 OXE_DEV void vl_group(u32x4 (&pf)[PF], int64_t g, int64_t g_next, const KqSegs &S, int nb, float *__restrict__ s,
                       const KqEpi &epi, uint8_t *wl, const uint32_t *yh, const float *yd, int *res) {
@@ -473,8 +473,13 @@ int vl_gemv_launch_nw(const KqSegs &S, int nb, const uint8_t *y, float *s, hipSt
 }
 // Four waves share the lanes' activations in LDS where staging them is what a workgroup spends its time on: at
 // least two lanes of rows of 2048 (Q3_K, whose waves need the most registers: 24 blocks in all; Q6_K also one lane of 3072).
-// Measured, one wave against four (us): Q4_K 8192 x 2048 2 lanes 11.4 / 9.4, 4 lanes 15.1 / 10.7, 100000 x 4096 4 lanes
-// 160 / 106; Q6_K 100000 x 3072 2 lanes 113 / 68; but one lane 700 x 2048 Q4_K 6.2 / 7.3, 100000 x 1024 24.3 / 27.1
+// Rows set no line: a few workgroups of four waves are still the shorter latency. Measured, one wave against four (us):
+//   Q4_K, 2048 long, 2 lanes: 32 rows 7.1 / 6.6, 512 7.0 / 7.0, 2048 7.7 / 6.7, 8192 10.7 / 9.0, 32768 19.7 / 19.0
+//   2048 x 4096, 2 / 4 lanes: Q3_K 12.2 / 9.9, 18.4 / 12.0; Q4_K 13.5 / 11.0, 18.8 / 12.5; Q5_K 15.1 / 12.7; Q6_K 15.0 / 12.2,
+//   20.8 / 14.4, one lane 12.3 / 10.8
+//   2048 x 2048, 4 lanes: Q3_K 10.5 / 7.6, Q4_K 10.5 / 7.6, Q5_K 10.9 / 8.2, Q6_K 10.4 / 7.8; 3 lanes Q3_K 9.1 / 7.3
+//   100000 rows: Q4_K 4096 long, 4 lanes 160 / 106; Q6_K 3072 long, 2 lanes 113 / 68
+// and the other side: one lane 700 x 2048 Q4_K 6.2 / 7.3, 100000 x 1024 24.3 / 27.1; Q5_K 512 x 2048, 2 lanes 7.5 / 7.8
 template <int TY, int NL, int PF>
 int vl_gemv_launch_pf(const KqSegs &S, int nb, const uint8_t *y, float *s, hipStream_t st, const KqEpi &epi) {
     if constexpr (PF >= 4 && (NL >= 2 || TY == 6)) {

@@ -22,10 +22,12 @@
 // from global memory, 32 rows apart per load, a single-wave workgroup ([2048 x 4096], 701 tokens, Q4_K) took 83 us against
 // 55. The tokens' codes go through LDS shared by the waves, 256 bytes a row per stage, double buffered, by direct
 // global-to-LDS loads; 128-byte code rows with their 16-byte chunks XOR-swizzled by f(r) = (r & 7) ^ ((r >> 3) & 1), as the
-// Q8_0 GEMM's. Bound by the VALU (unpacking, and the chain) at two waves per SIMD.
+// Q8_0 GEMM's. Bound by the VALU (unpacking, and the chain): in the largest launches it issues in 48 to 59 % of the
+// cycles (the Q8_0 GEMM's in 61 %), with the matrix cores busy 17 to 25 %, at two waves per SIMD (three for Q3_K; one for
+// single-wave workgroups).
 //
-// Measured, [12288 x 2048] over 2048 tokens with its quantisation: Q3_K 147 us, Q4_K 238, Q5_K 321, Q6_K 231.
-// A 701-token prompt through 8 layers of the Ornith file's types: 419 ms as decode runs of two positions, 5.1 ms.
+// Measured, 2048 tokens: [12352 x 2048] Q3_K 141 us, Q5_K 341, Q6_K 239; [9216 x 2048] Q4_K 165.
+// A 701-token prompt through 8 layers of the Ornith file's types: 419 ms as decode runs of two positions, 4.9 ms.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -82,7 +84,8 @@ struct Run {
 };
 
 // A block's bytes as a wave stages them: 32 rows, CH chunks of 16 bytes each, STRIDE bytes apart in LDS (8 consecutive
-// rows' 16-byte reads fall on distinct banks). Q3_K / Q6_K blocks (110 / 210 bytes) of odd index start 2 bytes past a
+// rows' 16-byte reads fall on distinct banks; the 4-byte reads behind them conflict, 13 % of Q3_K's LDS cycles and 29 % of
+// Q6_K's). Q6_K's 14 chunks end 12 bytes past its block: past the matrix's last block they read its allocation's margin. Q3_K / Q6_K blocks (110 / 210 bytes) of odd index start 2 bytes past a
 // dword (rows hold an even number of blocks): they are staged from the dword before, and read with that shift.
 template <int TY> struct Geo;
 template <> struct Geo<3> { static constexpr int BB = 110, CH = 7, STRIDE = 112; };

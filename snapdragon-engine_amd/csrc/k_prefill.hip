@@ -867,8 +867,8 @@ __global__ __launch_bounds__(PT) void entry_in_kernel(Q8W emb, const uint32_t *t
 // ---- host ----------------------------------------------------------------------------------------
 
 // prompts of at most this many positions of a model with K-quant / F32 matrices run as decode runs of two
-// positions (8 layers of the Ornith file's types: 2 positions 1.14 ms against 1.81 batched, 3 positions 2.28
-// against 1.57)
+// positions (as runs / batched, 40 layers: the Ornith file's types 2 positions 3.8 / 6.8 ms, 3 positions 7.0 / 6.9; the
+// Qwen3.6 file's 3.5 / 5.4 and 6.5 / 5.6)
 constexpr int PF_KQ_RUNS = 2;
 // a K-quant matrix and the column its rows start at
 struct KqPart {

@@ -7,7 +7,7 @@ A synthetic model with those types is written as a GGUF file (tests/gguf_writer.
 synthetic K-quant blocks); the engine created from the file must decode bit for bit like the
 oracle's typed engine on the same weights: prefill, logits, hidden states, host-driven MTP steps
 with accepted and rejected drafts, and device-driven steps. Such an engine runs per phase (the
-fused run kernel reads Q8_0 matrices only) and prefills two positions per run."""
+fused run kernel reads Q8_0 matrices only) and prefills three or more positions in one batched pass."""
 import os
 
 import numpy as np
@@ -74,7 +74,7 @@ def test_typed_engine_runs_per_phase_and_prefill_matches_oracle(typed_file):
         g.set_fused(True)   # the fused run kernel reads Q8_0 matrices only
     ref = O.Engine(d, seed=SEED, n_ctx=512, types=ty)
     toks = [int(v) % d.n_vocab for v in O.bench_prompt(9)]
-    print("prefill 9 tokens (two positions per run)", flush=True)
+    print("prefill 9 tokens (batched)", flush=True)
     nx, h = g.prefill(toks, hidden=True)
     want = [ref.step(t) for t in toks]
     assert nx == want[-1]

@@ -72,7 +72,7 @@ def test_kquant_projections_prefill_and_verify_match_oracle(typed_file):
     assert not g.fused
     ref = O.Engine(d, seed=SEED, n_ctx=512, types=ty)
     toks = [int(v) % d.n_vocab for v in O.bench_prompt(9)]
-    print("prefill 9 tokens (two positions per run)", flush=True)
+    print("prefill 9 tokens (batched)", flush=True)
     nx, h = g.prefill(toks, hidden=True)
     want = [ref.step(t) for t in toks]
     assert nx == want[-1]
