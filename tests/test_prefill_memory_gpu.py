@@ -1,5 +1,5 @@
-"""Device memory of the batched prefill: what its buffers hold as prompts grow, and what happens when they do not fit. The engine's own limit
-(oxe_engine_limit_bytes) stands in for a full device."""
+"""Device memory of the batched prefill: what its buffers hold as prompts grow, and what happens when they do
+not fit. The engine's own limit (oxe_engine_limit_bytes) stands in for a full device."""
 import numpy as np
 import pytest
 
