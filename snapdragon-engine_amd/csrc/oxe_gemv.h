@@ -170,8 +170,18 @@ inline int gemv_launch(int nl, const int8_t *wq, const uint16_t *wd, int64_t nro
                        Epi epi, hipStream_t st) {
     // at least 512 workgroups (two per CU) down to a quarter of the rows: a small matrix is one workgroup's
     // latency, and fewer rows shorten its chain phase (2 lanes: 4096 x 2048 6.2 -> 5.8 us, 700 x 2048 5.0 -> 3.7,
-    // 2048 x 512 3.1 -> 2.7)
+    // 2048 x 512 3.1 -> 2.7). Rows of 4096 (one to a pass of the workgroup): a quarter of the rows up to two
+    // workgroups per CU, all of them while they are one round of 256 workgroups (three lanes still a quarter: 1500 rows 8.1 / 8.1 /
+    // 7.7 us), then a quarter or (three lanes and more) half until that is 512 workgroups. Cold weights, all / half / a quarter of the rows, us: 1024 rows 1 lane 6.8 / 6.0 / 6.5, 4
+    // lanes 8.2 / 7.0 / 7.3; 1500 7.1 / 7.2 / 7.4, 8.4 / 8.5 / 8.8; 2048 7.2 / 7.3 / 8.2, 8.7 / 8.7 / 10.0; 3072 9.1 / 8.5 / 7.3,
+    // 9.6 / 8.5 / 9.2, 2 lanes 9.6 / 9.5 / 7.4; 4096 9.7 / 9.7 / 8.2, 10.1 / 9.6 / 10.6, 2 lanes 10.0 / 10.9 / 8.2; 6144 12.0 / 9.9
+    // / 12.9, 12.0 / 12.6 / 16.2, 2 lanes 10.9 / 11.3 / 13.2
     constexpr int R = GemvR<K>::R;
+    if (K == 4096 && nrows > 1024 && nrows <= 4096) {
+        if (nrows <= 2048 && nl != 3) return gemv_launch_r<K, R, Epi>(nl, wq, wd, nrows, a, isum_out, epi, st);
+        if (nrows > 2048 && nl > 2) return gemv_launch_r<K, R / 2, Epi>(nl, wq, wd, nrows, a, isum_out, epi, st);
+        return gemv_launch_r<K, R / 4, Epi>(nl, wq, wd, nrows, a, isum_out, epi, st);
+    }
     if (nrows >= 512 * R) return gemv_launch_r<K, R, Epi>(nl, wq, wd, nrows, a, isum_out, epi, st);
     if (nrows >= 256 * R) return gemv_launch_r<K, R / 2, Epi>(nl, wq, wd, nrows, a, isum_out, epi, st);
     return gemv_launch_r<K, R / 4, Epi>(nl, wq, wd, nrows, a, isum_out, epi, st);

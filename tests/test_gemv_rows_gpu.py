@@ -1,5 +1,5 @@
 """The Q8_0 GEMV's row counts per workgroup and its general-length kernel against the oracle, bit for bit: on both sides of
-the rules' lines (matrices of 2^19 weights; 256 and 512 workgroups), with a partial last workgroup, row lengths whose chunks
+the rules' lines (matrices of 2^19 weights; 256 and 512 workgroups; rows of 4096 at 1024, 2048 and 4096 rows), with a partial last workgroup, row lengths whose chunks
 straddle a workgroup's passes, and rows too long for the general kernel's LDS."""
 import numpy as np
 import pytest
@@ -12,7 +12,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("k,nr,nl", [(1120, 468, 3), (1120, 469, 3), (1120, 3001, 4), (96, 6001, 2), (8224, 70, 1), (15360, 40, 4),
                                      (3232, 1025, 2), (2048, 4095, 1), (2048, 8193, 2), (512, 8191, 4), (512, 16385, 1),
-                                     (4096, 2047, 3), (4096, 4097, 2), (65536, 9, 1), (32768, 17, 2)])
+                                     (4096, 2047, 3), (4096, 4097, 2), (65536, 9, 1), (32768, 17, 2),
+                                     (4096, 1024, 1), (4096, 1025, 2), (4096, 1025, 3), (4096, 2048, 4), (4096, 2049, 2), (4096, 2051, 3), (4096, 4096, 2),
+                                     (4096, 4095, 4)])
 def test_gemv_rows_bitexact(dev, k, nr, nl):
     import oxe_amd as A
     import torch
