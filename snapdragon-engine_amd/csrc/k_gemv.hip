@@ -125,7 +125,7 @@ static void gemv_any_launch(int64_t k, int64_t nr, int R, size_t lds, const int8
                        isum);
 }
 
-// Rows too long for that kernel's LDS, and matrices of at most 2^19 weights (700 x 320: 3.3 us against 3.7, the
+// Rows too long for that kernel's LDS or, with their lanes, for enough of its workgroups, and matrices of at most 2^19 weights (700 x 320: 3.3 us against 3.7, the
 // workgroup's phases cost more than its lines save): one wave per row; lane i forms the exact int32 dots of blocks i, i + 64, ...
 // for every activation lane, then thread l of the wave runs lane l's chain over the blocks.
 constexpr int GG_ROWS = 4;
@@ -183,7 +183,14 @@ int oxe_hip_gemv_q8_0(int64_t k, int64_t nr, int nl, const int8_t *wq, const uin
         R = (int)std::min<int64_t>(R, std::max<int64_t>(2, nr / 512));
         while (R > 1 && oxe::gemv_any_lds(k, nl, R) > 64 * 1024) R--;
         const size_t need = oxe::gemv_any_lds(k, nl, R);
-        if (nr * k > (1 << 19) && need <= 64 * 1024 && ((uintptr_t)wq | (uintptr_t)xq) % 16 == 0) {
+        // its workgroups stage the lanes' activations: over many rows that pays where the rows in flight on a CU, as many
+        // workgroups as its LDS holds, come to 43 KB. Against a wave per row, us: 8192 x 8192, 4 lanes (48 KB) 61 / 80, 9216 x 8192,
+        // 4 lanes (54) 69 / 91, 11008 x 8192, 3 lanes (43) 101 / 117 and
+        // x 4096 58 / 56, 18944 x 4096, 2 lanes (56) 96 / 91; but 12288 x 4096, 4 lanes (24) 100 / 59, 16384 x 4096, 3 lanes (32)
+        // 123 / 76, 12288 x 4096, 3 lanes (36) 72 / 59, 10240 x 4096, 4 lanes (40) 53 / 49. Up to 1536 rows its latency
+        // is the shorter one all the same (10240 x 1500, 4 lanes 26 / 34, 16384 x 1024, 3 lanes 39 / 50)
+        const bool pays = nr <= 1536 || (int64_t)(160 * 1024 / std::max<size_t>(1, need)) * R * k >= 43 * 1024;
+        if (nr * k > (1 << 19) && need <= 64 * 1024 && pays && ((uintptr_t)wq | (uintptr_t)xq) % 16 == 0) {
             const hipStream_t st = (hipStream_t)stream;
             if (nl == 1) oxe::gemv_any_launch<1>(k, nr, R, need, wq, wd, xq, xd, y, isum, st);
             else if (nl == 2) oxe::gemv_any_launch<2>(k, nr, R, need, wq, wd, xq, xd, y, isum, st);

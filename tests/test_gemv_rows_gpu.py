@@ -1,5 +1,6 @@
 """The Q8_0 GEMV's row counts per workgroup and its general-length kernel against the oracle, bit for bit: on both sides of
-the rules' lines (matrices of 2^19 weights; 256 and 512 workgroups; rows of 4096 at 1024, 2048 and 4096 rows), with a partial last workgroup, row lengths whose chunks
+the rules' lines (matrices of 2^19 weights; 256 and 512 workgroups; rows of 4096 at 1024, 2048 and 4096 rows;
+long rows of several lanes at 1536 rows), with a partial last workgroup, row lengths whose chunks
 straddle a workgroup's passes, and rows too long for the general kernel's LDS."""
 import numpy as np
 import pytest
@@ -13,8 +14,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("k,nr,nl", [(1120, 468, 3), (1120, 469, 3), (1120, 3001, 4), (96, 6001, 2), (8224, 70, 1), (15360, 40, 4),
                                      (3232, 1025, 2), (2048, 4095, 1), (2048, 8193, 2), (512, 8191, 4), (512, 16385, 1),
                                      (4096, 2047, 3), (4096, 4097, 2), (65536, 9, 1), (32768, 17, 2),
-                                     (4096, 1024, 1), (4096, 1025, 2), (4096, 1025, 3), (4096, 2048, 4), (4096, 2049, 2), (4096, 2051, 3), (4096, 4096, 2),
-                                     (4096, 4095, 4)])
+                                     (12288, 1536, 3), (12288, 1537, 3), (10240, 1537, 4), (8192, 1539, 4), (9216, 1537, 4),
+                                     (4096, 1024, 1), (4096, 1025, 2), (4096, 1025, 3), (4096, 2048, 4), (4096, 2049, 2), (4096, 2051, 3),
+                                     (4096, 4096, 2), (4096, 4095, 4)])
 def test_gemv_rows_bitexact(dev, k, nr, nl):
     import oxe_amd as A
     import torch
@@ -28,6 +30,27 @@ def test_gemv_rows_bitexact(dev, k, nr, nl):
     assert np.array_equal(isum.cpu().numpy(), isum_ref)
     assert np.array_equal(y.cpu().numpy().view(np.uint32), y_ref.view(np.uint32))
     assert torch.equal(A.gemv_q8_0(*args).view(torch.int32), y.view(torch.int32))
+
+
+@pytest.mark.parametrize("k,nr,nl", [(2048, 300, 2), (4096, 1500, 1), (1120, 3001, 3), (12288, 1537, 3), (320, 1000, 2)])
+def test_gemv_runs_on_the_callers_stream(dev, k, nr, nl):
+    """every route's launch is recorded by a capture of the current stream; replays give the eager bits"""
+    import oxe_amd as A
+    import torch
+    wq, wd = O.synth_q8(9, 61, O.T["OUTPUT"], nr, k)
+    xq, xd = O.quantize_q8_0(O.synth_normal(9, 61 * 64 + 41, nl * k).reshape(nl, k))
+    args = [_t(a, dev) for a in (wq, wd.view(np.int16), xq, xd.view(np.int16))]
+    want = A.gemv_q8_0(*args)
+    y = torch.zeros_like(want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        A.gemv_q8_0(*args, y=y)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int32), want.view(torch.int32))
 
 
 def test_quantize_row_tails(dev):
