@@ -38,8 +38,9 @@ OXE_API int oxe_hip_quantize_row_q8_0(const float *x, int64_t k, int64_t nrows, 
  * bit the per-lane GEMV; weights as int8 codes [nr][k] + fp16 scales [nr][k/32] (this build's
  * layout; see oxe_hip_repack_q8_0), lanes as produced by oxe_hip_quantize_row_q8_0; k any multiple
  * of 32 up to 131072 / nl (tuned kernels for 512, 2048 and 4096; otherwise workgroups of up to 16
- * rows, or a wave per row for matrices of at most 2^19 weights, rows too long for a workgroup's LDS,
- * many rows whose lanes leave it few workgroups, and arrays that are not 16-byte aligned). isum (optional, may be NULL): the exact int32 block dots [nl][nr][k/32].
+ * rows, or a wave per row for small matrices, for rows that with their lanes take too much of a
+ * workgroup's LDS, and for arrays that are not 16-byte aligned). isum (optional, may be NULL): the
+ * exact int32 block dots [nl][nr][k/32].
  * Replaces oxe_vl_gemv type 80 (lib.rs:113; csrc/oxe_vl.inc:78-107) with its return convention:
  * 1 = done, 0 = not handled with nothing written (nl outside 1..4, nr <= 0, k not a positive
  * multiple of 32 or past the limit), -2 launch error; and ggml_gemv_q8_0_4x8_q8_0 (lib.rs:75). */

@@ -125,8 +125,7 @@ static void gemv_any_launch(int64_t k, int64_t nr, int R, size_t lds, const int8
                        isum);
 }
 
-// Rows too long for that kernel's LDS or, with their lanes, for enough of its workgroups, and matrices of at most 2^19 weights (700 x 320: 3.3 us against 3.7, the
-// workgroup's phases cost more than its lines save): one wave per row; lane i forms the exact int32 dots of blocks i, i + 64, ...
+// Rows too long for that kernel's LDS or, with their lanes, for enough of its workgroups, and small matrices (700 x 320: 3.3 us against 3.7): one wave per row; lane i forms the exact int32 dots of blocks i, i + 64, ...
 // for every activation lane, then thread l of the wave runs lane l's chain over the blocks.
 constexpr int GG_ROWS = 4;
 __global__ __launch_bounds__(64 * GG_ROWS) void gemv_long_kernel(int64_t k, int64_t nr, int nl, const int8_t *__restrict__ wq,
@@ -190,7 +189,11 @@ int oxe_hip_gemv_q8_0(int64_t k, int64_t nr, int nl, const int8_t *wq, const uin
         // 123 / 76, 12288 x 4096, 3 lanes (36) 72 / 59, 10240 x 4096, 4 lanes (40) 53 / 49. Up to 1536 rows its latency
         // is the shorter one all the same (10240 x 1500, 4 lanes 26 / 34, 16384 x 1024, 3 lanes 39 / 50)
         const bool pays = nr <= 1536 || (int64_t)(160 * 1024 / std::max<size_t>(1, need)) * R * k >= 43 * 1024;
-        if (nr * k > (1 << 19) && need <= 64 * 1024 && pays && ((uintptr_t)wq | (uintptr_t)xq) % 16 == 0) {
+        // its phases cost more than its lines save on a small matrix: 2^19 weights, 7 * 2^17 where rows are short but
+        // hold a few blocks and the lanes are few (us, 2^19.3 weights: k 320, one lane 4.2 / 3.5, 448, four lanes 4.7 / 4.4; but k 160,
+        // three 4.1 / 4.1, 64, one 3.4 / 4.9, 768, one 3.9 / 4.4)
+        const int64_t small = k >= 128 && k <= 640 && 80 * nl <= k ? 7 << 17 : 1 << 19;
+        if (nr * k > small && need <= 64 * 1024 && pays && ((uintptr_t)wq | (uintptr_t)xq) % 16 == 0) {
             const hipStream_t st = (hipStream_t)stream;
             if (nl == 1) oxe::gemv_any_launch<1>(k, nr, R, need, wq, wd, xq, xd, y, isum, st);
             else if (nl == 2) oxe::gemv_any_launch<2>(k, nr, R, need, wq, wd, xq, xd, y, isum, st);

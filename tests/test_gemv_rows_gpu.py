@@ -1,5 +1,5 @@
 """The Q8_0 GEMV's row counts per workgroup and its general-length kernel against the oracle, bit for bit: on both sides of
-the rules' lines (matrices of 2^19 weights; 256 and 512 workgroups; rows of 4096 at 1024, 2048 and 4096 rows;
+the rules' lines (matrices of 2^19 and, of short rows, 7 * 2^17 weights; 256 and 512 workgroups; rows of 4096 at 1024, 2048 and 4096 rows;
 long rows of several lanes at 1536 rows), with a partial last workgroup, row lengths whose chunks
 straddle a workgroup's passes, and rows too long for the general kernel's LDS."""
 import numpy as np
@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("k,nr,nl", [(1120, 468, 3), (1120, 469, 3), (1120, 3001, 4), (96, 6001, 2), (8224, 70, 1), (15360, 40, 4),
                                      (3232, 1025, 2), (2048, 4095, 1), (2048, 8193, 2), (512, 8191, 4), (512, 16385, 1),
                                      (4096, 2047, 3), (4096, 4097, 2), (65536, 9, 1), (32768, 17, 2),
+                                     (320, 2867, 1), (320, 2868, 1), (320, 1876, 4), (160, 3751, 2), (160, 3751, 3), (448, 1500, 4),
                                      (12288, 1536, 3), (12288, 1537, 3), (10240, 1537, 4), (8192, 1539, 4), (9216, 1537, 4),
                                      (4096, 1024, 1), (4096, 1025, 2), (4096, 1025, 3), (4096, 2048, 4), (4096, 2049, 2), (4096, 2051, 3),
                                      (4096, 4096, 2), (4096, 4095, 4)])
